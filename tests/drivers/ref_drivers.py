@@ -71,7 +71,7 @@ def compile_driver(rel_src, exe, lattice=LATTICE, workdir=None, dev=True):
 
 def build():
     """Builds the drivers of RUN into tests/drivers/bin/; a no-op without the reference tree."""
-    if not os.path.isdir(REF) or not os.path.exists(LIB):
+    if not all(os.path.exists(os.path.join(REF, src)) for src, _ in RUN.values()) or not os.path.exists(LIB):
         return []
     os.makedirs(BIN, exist_ok=True)
     built = []
