@@ -37,7 +37,7 @@ struct AdjPhys {
 __device__ __forceinline__ double adj_g(const AdjPhys& p, double rho) {
     const double PI = 3.14159265358979323846;
     switch (p.interactions) {
-    case INT_UFG: return 0.37 * pow(3.0 * PI * PI * rho, 2.0 / 3.0) / 2.0;
+    case INT_UFG: return 0.37 * pow23(3.0 * PI * PI * rho) / 2.0;
     case INT_CONTACT: return 4 * PI * p.up[3] * rho;
     default: return 0.0;
     }

@@ -78,6 +78,41 @@ __device__ __forceinline__ cplx<R> cexp_(R re, R im) {
     return mk(t * c, t * s);
 }
 
+// x^(2/3) for x >= 0 (the unitary gas's density power; zero, infinity and NaN
+// are returned as they are, like pow's).  The argument is scaled by a power of
+// eight into [1/2, 8), so the whole range down to the denormals takes one
+// path; y ~ m^(-1/3) comes from the single-precision log2 / exp2 units to
+// ~4e-7 and enters once more through d = 1 - m y^3, formed without
+// cancellation from the low parts of its products:
+//   m^(2/3) = m y (1 - d)^(-1/3) = m y (1 + d/3 + 2 d^2/9 + ...)
+// The remaining terms are below 1e-13 (float, d^2) and 3e-19 (double, d^3).
+// Measured over the whole range against long double: at most 1.2e-7 and
+// 2.4e-16 relative (1 ulp), where pow with the exponent rounded to the type
+// reaches 2e-6 and 2.7e-14.  The passes of the unitary gas are bound by the
+// instructions of this power; with the library's pow a 128^3 complex64
+// friction step took 93.9 us, with this form 84.5 us, and a 64^3 complex64
+// gradient of 32 steps 6.62 -> 5.84 ms.
+__device__ __forceinline__ float pow23(float x) {
+    const int k = (__builtin_amdgcn_frexp_expf(x) * 21846) >> 16;  // a third of the exponent
+    const float m = __builtin_amdgcn_ldexpf(x, -3 * k);
+    const float y = __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(m) * -(1.0f / 3.0f));
+    const float t = m * y, tl = fmaf(m, y, -t);
+    const float p = y * y, pl = fmaf(y, y, -p);
+    const float d = fmaf(-t, p, 1.0f) - fmaf(t, pl, tl * p);
+    const float r = t + fmaf(t, d * (1.0f / 3.0f), tl);
+    return (x > 0.0f && x < __builtin_inff()) ? __builtin_amdgcn_ldexpf(r, 2 * k) : x;
+}
+__device__ __forceinline__ double pow23(double x) {
+    const int k = (__builtin_amdgcn_frexp_exp(x) * 21846) >> 16;
+    const double m = __builtin_amdgcn_ldexp(x, -3 * k);
+    // y has 24 bits, so y y is exact
+    const double y = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)m) * -(1.0f / 3.0f));
+    const double t = m * y, tl = fma(m, y, -t), p = y * y;
+    const double d = fma(-t, p, 1.0) - tl * p;
+    const double r = t + fma(t, d * fma(d, 2.0 / 9.0, 1.0 / 3.0), tl);
+    return (x > 0.0 && x < __builtin_inf()) ? __builtin_amdgcn_ldexp(r, 2 * k) : x;
+}
+
 constexpr int kMaxUserParams = 32;
 
 // Physics codes: INTERACTIONS (dev/gpe_user_defined.h:90,169,276,356) and
@@ -206,7 +241,7 @@ __device__ __forceinline__ R dedfdn(const Phys<R>& p, R rho, unsigned it, unsign
     }
     switch (p.interactions) {
     case INT_UFG:
-        return (R)0.37 * g_pow((R)3.0 * PI * PI * rho, (R)(2.0 / 3.0)) / (R)2.0;
+        return (R)0.37 * pow23((R)3.0 * PI * PI * rho) / (R)2.0;
     case INT_ETF: {
         const R XI = (R)0.37, CT = (R)0.901;
         const R a = p.up[3];
@@ -238,7 +273,7 @@ __device__ __forceinline__ double edf(const Phys<R>& p, const double* up, double
     }
     switch (p.interactions) {
     case INT_UFG:
-        return 0.37 * 0.6 * rho * pow(3.0 * PI * PI * rho, 2.0 / 3.0) / 2.;
+        return 0.37 * 0.6 * rho * pow23(3.0 * PI * PI * rho) / 2.;
     case INT_ETF: {
         const double XI = 0.37, CT = 0.901;
         const double a = up[3];
