@@ -421,7 +421,13 @@ __device__ __forceinline__ void fft_stages(cplx<T>* lds, const TwE<T>* tw) {
 
 // ------------------------------------------------------ pass arguments
 
-enum LoadMode { LOAD_PLAIN = 0, LOAD_PSI0 = 1, LOAD_PART2 = 2 };
+// (3 is LOAD_REDPOT of the z-wave passes)
+enum LoadMode {
+    LOAD_PLAIN = 0,
+    LOAD_PSI0 = 1,
+    LOAD_PART2 = 2,
+    LOAD_RHO = 4,  // psi (rescaled with F_SCALE) -> its density as a complex value (dev/gpe_engine.cu:618-626)
+};
 enum MidMode {
     MID_NONE = 0,
     MID_EXPT = 1,        // kinetic factor Kx Ky Kz/N (orginal/gpe_engine.cu:880-895)
@@ -439,6 +445,9 @@ enum MidMode {
     // the kinetic factor split by axis, K = (K_y K_z) K_x: K_y K_z in a y
     // turn-around whose data is already in k_z, K_x in the x turn-around
     MID_EXPT_SEP = 13,
+    MID_DIP_STEP = 14,   // psi exp(c (Vext + Vdip)), Vdip the real part of the value (dev/gpe_engine.cu:984-1008)
+    MID_DIP_RHO = 15,    // psi stored, its density goes on (dev/gpe_engine.cu:618-626)
+    MID_DIP_E2 = 16,     // sum rho Vdip (dev/gpe_engine.cu:1768-1782)
 };
 
 // Fourier transform of the particle-particle potential of z-polarised dipoles
@@ -462,6 +471,7 @@ enum PassFlags {
     F_NEXT_PSI = 128,     // MID_VSTEP3: continue with the next step's psi0 (QF transform)
     F_IMPRINT_NEXT = 256, // MID_VSTEP3: imprint the next step's psi0
     F_IMPRINT_MID = 512,  // LOAD_PART2: re-imprint psi0 before the corrector (ITE vortex)
+    F_TWICE = 1024,       // MID_DIP_STEP: the half steps on both sides of a step boundary in one factor
 };
 
 template <typename T>
@@ -764,6 +774,12 @@ __device__ __forceinline__ cplx<T> load_op_m(const PassArgs<T>& a, const ElemIn<
             v = mul_exp(v, a.ph.c.x * lv, a.ph.c.y * lv);
         }
         return v;
+    } else if constexpr (LM == LOAD_RHO) {
+        if (a.flags & F_SCALE) {
+            v = cscale(v, (T)a.scal[1]);
+            a.psiA[off] = v;
+        }
+        return mk((T)dens64((double)a.ph.gamma, (double)v.x, (double)v.y), (T)0);
     } else {
         // LOAD_PART2: v is the predictor phi3 (orginal/gpe_engine.cu:817-868)
         cplx<T> phi3 = v;
@@ -784,6 +800,7 @@ template <bool UH, typename T>
 __device__ __forceinline__ cplx<T> load_op2(const PassArgs<T>& a, const ElemIn<T>& e, cplx<T> v, double* acc) {
     if (a.load_mode == LOAD_PLAIN) return load_op_m<LOAD_PLAIN, UH>(a, e, v, acc);
     if (a.load_mode == LOAD_PSI0) return load_op_m<LOAD_PSI0, UH>(a, e, v, acc);
+    if (a.load_mode == LOAD_RHO) return load_op_m<LOAD_RHO, UH>(a, e, v, acc);
     return load_op_m<LOAD_PART2, UH>(a, e, v, acc);
 }
 
@@ -848,6 +865,18 @@ __device__ __forceinline__ cplx<T> mid_op_m(const PassArgs<T>& a, const ElemIn<T
         const cplx<T> p = e.aux;
         a.rout[off] = (double)(p.x * v.x + p.y * v.y);
         return v;
+    } else if constexpr (MM == MID_DIP_STEP) {
+        const cplx<T> l = modify_at<UH>(a, e, e.aux, e.it);
+        const T lv = (e.vx + v.x) * ((a.flags & F_TWICE) ? (T)2 : (T)1);
+        const cplx<T> r = mul_exp(l, a.ph.c.x * lv, a.ph.c.y * lv);
+        if (a.flags & F_RED_NORM) acc[0] += dens64((double)a.ph.gamma, (double)r.x, (double)r.y);
+        return r;
+    } else if constexpr (MM == MID_DIP_RHO) {
+        a.psiA[off] = v;
+        return mk((T)dens64((double)a.ph.gamma, (double)v.x, (double)v.y), (T)0);
+    } else if constexpr (MM == MID_DIP_E2) {
+        acc[0] += dens64((double)a.ph.gamma, (double)e.aux.x, (double)e.aux.y) * (double)v.x;
+        return v;
     } else if constexpr (MM == MID_EXPT || MM == MID_EXPTC || MM == MID_K2 || MM == MID_KA || MM == MID_VPP ||
                          MM == MID_EXPT_SEP) {
         return mid_op_lean(a, e.c, v);
@@ -866,6 +895,9 @@ __device__ __forceinline__ cplx<T> mid_op2(const PassArgs<T>& a, const ElemIn<T>
     case MID_KIN_SUM: return mid_op_m<MID_KIN_SUM, UH>(a, e, v, acc);
     case MID_VPP_SUM: return mid_op_m<MID_VPP_SUM, UH>(a, e, v, acc);
     case MID_OVERLAP_RE: return mid_op_m<MID_OVERLAP_RE, UH>(a, e, v, acc);
+    case MID_DIP_STEP: return mid_op_m<MID_DIP_STEP, UH>(a, e, v, acc);
+    case MID_DIP_RHO: return mid_op_m<MID_DIP_RHO, UH>(a, e, v, acc);
+    case MID_DIP_E2: return mid_op_m<MID_DIP_E2, UH>(a, e, v, acc);
     case MID_EXPT:
     case MID_EXPTC:
     case MID_K2:
@@ -1440,7 +1472,8 @@ struct FullLds {
 template <typename T>
 __device__ __forceinline__ bool needs_psi0(const PassArgs<T>& a) {
     return a.load_mode == LOAD_PART2 || a.mid_mode == MID_VSTEP2 || a.mid_mode == MID_PART1 ||
-           a.mid_mode == MID_QF_VSTEP1 || a.mid_mode == MID_OVERLAP_RE;
+           a.mid_mode == MID_QF_VSTEP1 || a.mid_mode == MID_OVERLAP_RE || a.mid_mode == MID_DIP_STEP ||
+           a.mid_mode == MID_DIP_E2;
 }
 template <typename T>
 __device__ __forceinline__ const T* real_side(const PassArgs<T>& a) {
@@ -1517,7 +1550,7 @@ __device__ __forceinline__ void full_body(const PassArgs<T>& a, FullLds<T, N, CO
     }
 
     // gather: unrolled plain loads of every input of the tile
-    const cplx<T>* msrc = (a.load_mode == LOAD_PSI0) ? a.psiA : a.src;
+    const cplx<T>* msrc = (a.load_mode == LOAD_PSI0 || a.load_mode == LOAD_RHO) ? a.psiA : a.src;
     const bool want_psi0 = CONTIG && needs_psi0(a);
     const T* rsrc = CONTIG ? real_side(a) : nullptr;
 #pragma unroll

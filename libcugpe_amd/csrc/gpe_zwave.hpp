@@ -308,7 +308,7 @@ void zwave_kernel(const PassArgs<T> a) {
     // inactive lanes (past the last pencil) read pencil 0 and store nothing
     cplx<T> v[B];
     {
-        const cplx<T>* src = (LM == LOAD_PSI0) ? a.psiA : a.src;
+        const cplx<T>* src = (LM == LOAD_PSI0 || LM == LOAD_RHO) ? a.psiA : a.src;
 #pragma unroll
         for (int b = 0; b < B; b++) v[b] = src[base + (unsigned)(A * b)];
     }
@@ -332,13 +332,15 @@ void zwave_kernel(const PassArgs<T> a) {
     constexpr bool PRE = (LM != LOAD_PLAIN);   // physics before the first transform
     constexpr bool POST = (MM != MID_NONE);    // physics after it
     constexpr bool NEED_AUX = (LM == LOAD_PART2) || MM == MID_VSTEP2 || MM == MID_PART1 ||
-                              MM == MID_QF_VSTEP1 || MM == MID_OVERLAP_RE;
+                              MM == MID_QF_VSTEP1 || MM == MID_OVERLAP_RE || MM == MID_DIP_STEP ||
+                              MM == MID_DIP_E2;
     const T* rs = real_side(a);
     const bool qf = (a.flags & F_QF) != 0;
     // the fast chunk forms: ops without imprint, built-in physics
     const bool fast = (MM == MID_VSTEP2) || (MM == MID_VSTEP3 && !(a.flags & F_IMPRINT_NEXT)) ||
                       (LM == LOAD_PSI0 && !(a.flags & F_IMPRINT)) || (LM == LOAD_PART2 && !(a.flags & F_IMPRINT_MID)) ||
-                      MM == MID_PART1 || MM == MID_QF_VSTEP1;
+                      MM == MID_PART1 || MM == MID_QF_VSTEP1 || LM == LOAD_RHO || MM == MID_DIP_STEP ||
+                      MM == MID_DIP_RHO || MM == MID_DIP_E2;
     cplx<T> ax[2][CH];
     T rx[2][CH];
     auto fetch = [&](int q, int slot) __attribute__((always_inline)) {
@@ -391,6 +393,47 @@ void zwave_kernel(const PassArgs<T> a) {
 #pragma unroll
                     for (int j = 0; j < CH; j++) lv[j] = vx[j] + gv[j] + (qf ? rx[slot][j] : (T)0);
                     mul_exp_chunk(u, lv, a.ph.c.x, a.ph.c.y);
+                }
+            } else if constexpr (LM == LOAD_RHO) {
+                if (a.flags & F_SCALE) {
+                    const T f = (T)a.scal[1];
+#pragma unroll
+                    for (int j = 0; j < CH; j++) u[j] = cscale(u[j], f);
+                    if (ok) {
+#pragma unroll
+                        for (int j = 0; j < CH; j++) st_nt(&a.psiA[off_of(q * CH + j)], u[j]);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < CH; j++)
+                    u[j] = mk((T)dens64((double)a.ph.gamma, (double)u[j].x, (double)u[j].y), (T)0);
+            } else if constexpr (MM == MID_DIP_RHO) {
+                // the wave function after the kinetic factor, then its density
+                if (ok) {
+#pragma unroll
+                    for (int j = 0; j < CH; j++) st_nt(&a.psiA[off_of(q * CH + j)], u[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < CH; j++)
+                    u[j] = mk((T)dens64((double)a.ph.gamma, (double)u[j].x, (double)u[j].y), (T)0);
+            } else if constexpr (MM == MID_DIP_STEP) {
+                // potential half step with the convolution potential (dev/gpe_engine.cu:984-1008)
+                const T two = (a.flags & F_TWICE) ? (T)2 : (T)1;
+#pragma unroll
+                for (int j = 0; j < CH; j++) {
+                    lv[j] = (vx[j] + u[j].x) * two;
+                    u[j] = ax[slot][j];
+                }
+                mul_exp_chunk(u, lv, a.ph.c.x, a.ph.c.y);
+                if ((a.flags & F_RED_NORM) && ok) {
+#pragma unroll
+                    for (int j = 0; j < CH; j++) acc[0] += dens64((double)a.ph.gamma, (double)u[j].x, (double)u[j].y);
+                }
+            } else if constexpr (MM == MID_DIP_E2) {
+                if (ok) {
+#pragma unroll
+                    for (int j = 0; j < CH; j++)
+                        acc[0] += dens64((double)a.ph.gamma, (double)ax[slot][j].x, (double)ax[slot][j].y) * (double)u[j].x;
                 }
             } else if constexpr (MM == MID_VSTEP2) {
                 // predictor end and corrector potential (orginal/gpe_engine.cu:774-801)
@@ -568,6 +611,11 @@ unsigned launch_zwave(const PassArgs<T>& a, hipStream_t s) {
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_VSTEP2)
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_VSTEP3)
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_QF_VSTEP1)
+        GPE_ZW(SHAPE_F, LOAD_RHO, MID_NONE)
+        GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_DIP_STEP)
+        GPE_ZW(SHAPE_I, LOAD_PLAIN, MID_DIP_STEP)
+        GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_DIP_RHO)
+        GPE_ZW(SHAPE_I, LOAD_PLAIN, MID_DIP_E2)
 #undef GPE_ZW
         return 0;
     }
