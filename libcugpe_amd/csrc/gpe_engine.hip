@@ -88,10 +88,12 @@ struct gpe_engine_s {
     // adjoint of a real-time run (gpe_engine_adjoint_forward / _backward)
     void *adj_ck = nullptr, *adj_seg = nullptr;  // checkpoints, one segment of states
     size_t adj_ck_len = 0, adj_seg_len = 0;     // in states
-    void *adj_lam = nullptr, *adj_phi = nullptr, *adj_lam0 = nullptr, *adj_tgt = nullptr, *adj_fin = nullptr;
+    void *adj_lam = nullptr, *adj_lam0 = nullptr, *adj_tgt = nullptr, *adj_fin = nullptr;
+    void* adj_phi = nullptr;      // predictor ends of a segment's steps, or of one step (adj_phi_len in states)
+    size_t adj_phi_len = 0;
+    void *adj_Ktab = nullptr, *adj_Khl = nullptr;  // conjugate kinetic factors
     double *adj_vb = nullptr, *adj_grad = nullptr, *adj_vx = nullptr;
     int adj_nt = 0, adj_C = 0;
-    unsigned adj_it0 = 0;
     bool adj_ready = false;
     unsigned adj_gen = 0;  // gen at the forward run: a parameter change since then voids the backward run
     double adj_fr = 0, adj_fi = 0;  // lambda(T) = (fr + i fi) psi_target
@@ -173,13 +175,15 @@ void build_kinetic(gpe_engine_s* e) {
 
 // Kinetic factors in FP64; for complex64 also K_x and the products K_y K_z
 // per (iy, iz), each as a float pair hi + lo with hi + lo = K to ~1e-15.
-int upload_kinetic(gpe_engine_s* e) {
+// conj: the conjugate tables (the adjoint's kinetic step) into the adjoint's
+// own arrays.
+int upload_kinetic_tables(gpe_engine_s* e, bool conj) {
+    auto val = [&](std::complex<double> v) { return conj ? std::conj(v) : v; };
     std::vector<cplx<double>> K;
-    for (auto& v : e->Kx) K.push_back(mk(v.real(), v.imag()));
-    for (auto& v : e->Ky) K.push_back(mk(v.real(), v.imag()));
-    for (auto& v : e->Kz) K.push_back(mk(v.real(), v.imag()));
+    for (const auto* t : {&e->Kx, &e->Ky, &e->Kz})
+        for (auto& v : *t) K.push_back(mk(val(v).real(), val(v).imag()));
     HIP_TRY(hipStreamSynchronize(e->stream));
-    HIP_TRY(hipMemcpy(e->Ktab, K.data(), K.size() * sizeof(cplx<double>), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(conj ? e->adj_Ktab : e->Ktab, K.data(), K.size() * sizeof(cplx<double>), hipMemcpyHostToDevice));
     if (e->Khl) {
         std::vector<cplx<float>> h;
         h.reserve(2 * ((size_t)e->nx + (size_t)e->ny * e->nz));
@@ -188,12 +192,17 @@ int upload_kinetic(gpe_engine_s* e) {
             h.push_back(mk(hr, hi));
             h.push_back(mk((float)(v.real() - (double)hr), (float)(v.imag() - (double)hi)));
         };
-        for (auto& v : e->Kx) split(v);
+        for (auto& v : e->Kx) split(val(v));
         for (int iy = 0; iy < e->ny; iy++)
-            for (int iz = 0; iz < e->nz; iz++) split(e->Ky[iy] * e->Kz[iz]);
-        HIP_TRY(hipMemcpy(e->Khl, h.data(), h.size() * sizeof(cplx<float>), hipMemcpyHostToDevice));
+            for (int iz = 0; iz < e->nz; iz++) split(val(e->Ky[iy] * e->Kz[iz]));
+        HIP_TRY(hipMemcpy(conj ? e->adj_Khl : e->Khl, h.data(), h.size() * sizeof(cplx<float>), hipMemcpyHostToDevice));
     }
     return 0;
+}
+
+int upload_kinetic(gpe_engine_s* e) {
+    if (int r = upload_kinetic_tables(e, false)) return r;
+    return e->adj_Ktab ? upload_kinetic_tables(e, true) : 0;
 }
 
 template <typename T>
@@ -376,9 +385,13 @@ int normalize_t(gpe_engine_s* e) {
 // step but the last ends in a pass that also opens the next one.
 // pin: 0 none, 1 vortex imprint, 2 imprint where |psi| > 1e-15, 3 stored phase;
 // mid_pin: re-applied after the predictor normalisation in imaginary time
+// psi0, psi1, phi3 (real time without pinning or friction): where the step reads its state,
+// leaves it, and stores its predictor end; null: in psi, in psi, not at all.
+// psi is then the corrector's work array.
 struct StepPlan {
     int pin = 0;
     bool mid_pin = false;
+    void *psi0 = nullptr, *psi1 = nullptr, *phi3 = nullptr;
 };
 
 template <typename T>
@@ -390,6 +403,15 @@ PassArgs<T> step_args(gpe_engine_s* e, const StepPlan& sp) {
     // user hooks read the step's time index from device memory, so that a
     // captured step graph stays valid for every step it is replayed for
     if (e->uses_hooks) a.ph.itp = e->itdev;
+    if (sp.psi0) a.psiA = (cplx<T>*)sp.psi0;
+    a.phi3 = (cplx<T>*)sp.phi3;
+    return a;
+}
+
+// the arguments of the pass that ends the step: its state goes to psi1
+template <typename T>
+PassArgs<T> end_args(const gpe_engine_s* e, PassArgs<T> a, const StepPlan& sp) {
+    a.psiA = (cplx<T>*)(sp.psi1 ? sp.psi1 : e->A);
     return a;
 }
 
@@ -462,10 +484,11 @@ void issue_step(gpe_engine_s* e, const StepPlan& sp, bool last) {
         const PassArgs<T> a = step_args<T>(e, sp);
         void *A = e->A, *B = e->B;
         run_pass<T>(e, a, {0, B, B, -1, +1, LOAD_PLAIN, MID_EXPT_SEP, STORE_PLAIN, 0, 0});
-        plane_run<T>(e, a, PL_VSTEP2, B, A, 0);
+        plane_run<T>(e, a, sp.phi3 ? PL_VSTEP2P : PL_VSTEP2, B, A, 0);
         run_pass<T>(e, a, {0, A, A, -1, +1, LOAD_PLAIN, MID_EXPT_SEP, STORE_PLAIN, 0, 0});
-        if (!last) plane_run<T>(e, a, PL_VSTEP3_NEXT, A, B, F_NEXT_VSTEP1);
-        else plane_run<T>(e, a, PL_VSTEP3_LAST, A, nullptr, 0);
+        const PassArgs<T> a1 = end_args<T>(e, a, sp);
+        if (!last) plane_run<T>(e, a1, PL_VSTEP3_NEXT, A, B, F_NEXT_VSTEP1);
+        else plane_run<T>(e, a1, PL_VSTEP3_LAST, A, nullptr, 0);
         if (e->uses_hooks) launch_tick(e->itdev, e->stream);
         return;
     }
@@ -486,7 +509,7 @@ void issue_step(gpe_engine_s* e, const StepPlan& sp, bool last) {
     // predictor kinetic step of phi1
     kinetic_kz<T>(e, a, B);
     if (!ite) {
-        run_pass<T>(e, a, {2, B, A, I, F, LOAD_PLAIN, MID_VSTEP2, STORE_PLAIN, fqf, 0});
+        run_pass<T>(e, a, {2, B, A, I, F, LOAD_PLAIN, sp.phi3 ? MID_VSTEP2P : MID_VSTEP2, STORE_PLAIN, fqf, 0});
     } else {
         const int nb = run_pass<T>(e, a, {2, B, B, I, 0, LOAD_PLAIN, MID_PART1, STORE_PLAIN, fqf, 1});
         finalize(e, nb, 1, FIN_NORM, 0, 1.0);
@@ -498,9 +521,9 @@ void issue_step(gpe_engine_s* e, const StepPlan& sp, bool last) {
     if (!ite) {
         if (!last) {
             const int nxt = (qf ? F_NEXT_PSI : F_NEXT_VSTEP1) | (vortex ? F_IMPRINT_NEXT : 0);
-            run_pass<T>(e, a, {2, A, qf ? C : B, I, F, LOAD_PLAIN, MID_VSTEP3, STORE_PLAIN, nxt, 0});
+            run_pass<T>(e, end_args<T>(e, a, sp), {2, A, qf ? C : B, I, F, LOAD_PLAIN, MID_VSTEP3, STORE_PLAIN, nxt, 0});
         } else {
-            run_pass<T>(e, a, {2, A, nullptr, I, 0, LOAD_PLAIN, MID_VSTEP3, STORE_NONE, 0, 0});
+            run_pass<T>(e, end_args<T>(e, a, sp), {2, A, nullptr, I, 0, LOAD_PLAIN, MID_VSTEP3, STORE_NONE, 0, 0});
         }
     } else {
         const int nb = run_pass<T>(e, a, {2, A, nullptr, I, 0, LOAD_PLAIN, MID_VSTEP3, STORE_NONE, F_RED_NORM, 1});
@@ -669,9 +692,9 @@ int currents_t(gpe_engine_s* e, double* js[3]) {
     return 0;
 }
 
+// n host complex128 values into a device array of the working precision
 template <typename T>
-int set_psi_t(gpe_engine_s* e, const cuCplx* psi, size_t inst = 0) {
-    cplx<T>* dst = (cplx<T>*)e->A + inst * e->n;
+int from_host(gpe_engine_s* e, const cuCplx* psi, cplx<T>* dst) {
     if (sizeof(T) == sizeof(double)) {
         HIP_TRY(hipMemcpyAsync(dst, psi, e->n * sizeof(cuCplx), hipMemcpyHostToDevice, e->stream));
     } else {
@@ -687,6 +710,11 @@ int set_psi_t(gpe_engine_s* e, const cuCplx* psi, size_t inst = 0) {
     }
     HIP_TRY(hipStreamSynchronize(e->stream));
     return 0;
+}
+
+template <typename T>
+int set_psi_t(gpe_engine_s* e, const cuCplx* psi, size_t inst = 0) {
+    return from_host<T>(e, psi, (cplx<T>*)e->A + inst * e->n);
 }
 
 template <typename T>
@@ -715,7 +743,7 @@ void free_all(gpe_engine_s* e) {
                     e->twlo[2], e->Ktab, e->ktab, e->Khl, e->vtab,
                     e->k64, e->updev, e->itdev, e->partials, e->scal, e->rout, e->phase, e->wind, e->adj_ck, e->adj_seg,
                     e->adj_lam, e->adj_phi, e->adj_lam0, e->adj_tgt, e->adj_fin, e->adj_vb, e->adj_grad,
-                    e->adj_vx};
+                    e->adj_vx, e->adj_Ktab, e->adj_Khl};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& ev : e->prof_ev) {
@@ -1527,7 +1555,7 @@ int gpe_engine_energy_dipolar(gpe_engine_t e, int method, double* t, double* edi
 // ====================================================================== adjoint
 //
 // Gradient of L = 1 - |<psi_t|psi(T)>|^2 / (|psi_t|^2 |psi(0)|^2) with respect
-// to V_ext at every point for nt real-time steps (gpe_adjoint.hip holds the
+// to V_ext at every point for nt real-time steps (gpe_adjoint.hpp holds the
 // pointwise parts and the derivation).  The forward run keeps the state every
 // C steps (C = ceil(sqrt(nt)) by default); the backward run recomputes one
 // segment of C states at a time from its checkpoint and walks it backwards:
@@ -1545,34 +1573,59 @@ int adj_alloc(void** p, size_t* have, size_t want, size_t unit) {
     return 0;
 }
 
-// psi <- K psi (adjoint: conj K) on a buffer, in place
-template <typename T>
-void kinetic_apply(gpe_engine_s* e, void* buf, bool adjoint) {
-    PassArgs<T> a = base_args<T>(e);
-    run_pass<T>(e, a, {2, buf, buf, -1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
-    run_pass<T>(e, a, {1, buf, buf, -1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
-    run_pass<T>(e, a, {0, buf, buf, -1, 1, LOAD_PLAIN, adjoint ? MID_EXPTC : MID_EXPT, STORE_PLAIN, 0, 0});
-    run_pass<T>(e, a, {1, buf, buf, 1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
-    run_pass<T>(e, a, {2, buf, buf, 1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
+// nt real-time steps from the state at `from`: step j leaves its state at
+// to(j) and its predictor end at phi(j) (null: not stored)
+template <typename T, typename To, typename Phi>
+void adj_steps(gpe_engine_s* e, int nt, void* from, To&& to, Phi&& phi) {
+    StepPlan sp;
+    sp.psi0 = from;
+    issue_open<T>(e, sp);
+    for (int j = 0; j < nt; j++) {
+        sp.psi1 = to(j);
+        sp.phi3 = phi(j);
+        issue_step<T>(e, sp, j == nt - 1);
+        sp.psi0 = sp.psi1;
+    }
 }
 
 template <typename T>
-AdjArgs adj_args(gpe_engine_s* e) {
-    AdjArgs a;
+AdjArgs<T> adj_args(gpe_engine_s* e) {
+    AdjArgs<T> a;
     std::memset(&a, 0, sizeof(a));
-    a.interactions = e->interactions;
-    a.gamma = e->gamma;
-    for (int i = 0; i < kMaxUserParams; i++) a.up[i] = e->up[i];
-    a.cx = e->c.real();
-    a.cy = e->c.imag();
+    a.p.interactions = e->interactions;
+    a.p.gamma = e->gamma;
+    a.p.a = e->up[3];
+    a.p.cx = e->c.real();
+    a.p.cy = e->c.imag();
     a.n = e->n;
     a.vx = e->adj_vx;
-    a.phi = e->adj_phi;
-    a.lam = e->adj_lam;
-    a.lam0 = e->adj_lam0;
+    a.lam = (cplx<T>*)e->adj_lam;
+    a.lam0 = (cplx<T>*)e->adj_lam0;
     a.vb = e->adj_vb;
     a.grad = e->adj_grad;
+    a.tw = (const cplx<T>*)e->tw[2];
+    a.twlo = (const cplx<T>*)e->twlo[2];
+    a.M = (unsigned)(e->n / (size_t)e->nz);
     return a;
+}
+
+// One z pass of a backward step: in wave registers, or its parts as pointwise
+// kernels between plain z passes (no wave split for the length, or launcher
+// variant bit 0)
+template <typename T>
+void adj_zpass(gpe_engine_s* e, const AdjArgs<T>& a, int pass) {
+    if (!(e->variant & 1) && launch_adjoint_z<T>(e->nz, a, pass, e->stream)) return;
+    const PassArgs<T> b = base_args<T>(e);
+    if (pass != ADJ_P2) run_pass<T>(e, b, {2, a.lam, a.lam, 1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
+    launch_adjoint_point<T>(a, pass == ADJ_P4P2 ? ADJ_P4 : pass, e->stream);
+    if (pass == ADJ_P4P2) {
+        AdjArgs<T> c = a;
+        c.psi1 = a.psi0;
+        c.psi0 = a.psi0p;
+        c.phi3 = a.phi3p;
+        launch_adjoint_point<T>(c, ADJ_P2, e->stream);
+    }
+    if (pass != ADJ_P4) run_pass<T>(e, b, {2, a.lam, a.lam, -1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
 }
 
 template <typename T>
@@ -1584,7 +1637,7 @@ int adjoint_forward_t(gpe_engine_s* e, int nt, const cuCplx* tgt, int ckpt, doub
     e->adj_ready = false;
     int r = adj_alloc(&e->adj_ck, &e->adj_ck_len, (size_t)nck * n, cs);
     if (!r) r = adj_alloc(&e->adj_seg, &e->adj_seg_len, (size_t)(C + 1) * n, cs);
-    for (void** p : {&e->adj_lam, &e->adj_phi, &e->adj_lam0, &e->adj_tgt, &e->adj_fin}) {
+    for (void** p : {&e->adj_lam, &e->adj_lam0, &e->adj_tgt, &e->adj_fin}) {
         have = *p ? n : 0;
         if (!r) r = adj_alloc(p, &have, n, cs);
     }
@@ -1593,22 +1646,29 @@ int adjoint_forward_t(gpe_engine_s* e, int nt, const cuCplx* tgt, int ckpt, doub
         if (!r) r = adj_alloc((void**)p, &have, n, sizeof(double));
     }
     if (r) return r;
+    if (!e->adj_Ktab) {
+        HIP_TRY(hipMalloc(&e->adj_Ktab, (size_t)(e->nx + e->ny + e->nz) * sizeof(cplx<double>)));
+        if (e->Khl) HIP_TRY(hipMalloc(&e->adj_Khl, 2 * ((size_t)e->nx + (size_t)e->ny * e->nz) * sizeof(cplx<float>)));
+        if (int q = upload_kinetic_tables(e, true)) return q;
+    }
+    // the predictor ends of a whole segment, or, where they do not fit, of
+    // one step (then each is computed again from its step's input)
+    if (adj_alloc(&e->adj_phi, &e->adj_phi_len, (size_t)C * n, cs)) {
+        (void)hipGetLastError();
+        if ((r = adj_alloc(&e->adj_phi, &e->adj_phi_len, n, cs))) return r;
+    }
     // target in the working precision, V_ext as the forward kernels see it
-    {
-        std::vector<cplx<T>> t(n);
-        for (size_t i = 0; i < n; i++) t[i] = mk((T)tgt[i].x, (T)tgt[i].y);
-        HIP_TRY(hipMemcpyAsync(e->adj_tgt, t.data(), n * cs, hipMemcpyHostToDevice, e->stream));
-        HIP_TRY(hipStreamSynchronize(e->stream));
-    }
+    if ((r = from_host<T>(e, tgt, (cplx<T>*)e->adj_tgt))) return r;
     launch_adjoint_vfill<T>(base_args<T>(e).ph, e->adj_vx, n, e->stream);
-    e->adj_it0 = e->it;
-    for (int k = 0; k < nt; k++) {
-        if (k % C == 0)
-            HIP_TRY(hipMemcpyAsync((char*)e->adj_ck + (size_t)(k / C) * n * cs, e->A, n * cs, hipMemcpyDeviceToDevice,
-                                   e->stream));
-        r = evolve_t<T>(e, 1, nullptr, 0, false);
-        if (r) return r;
-    }
+    HIP_TRY(hipMemcpyAsync(e->adj_ck, e->A, n * cs, hipMemcpyDeviceToDevice, e->stream));
+    adj_steps<T>(
+        e, nt, e->A,
+        [&](int j) -> void* {
+            const int k = j + 1;  // the state's time index
+            return (k % C == 0 && k < nt) ? (char*)e->adj_ck + (size_t)(k / C) * n * cs : (char*)e->A;
+        },
+        [](int) -> void* { return nullptr; });
+    e->it += (unsigned)nt;
     const int nb = launch_adjoint_overlap<T>(e->A, e->adj_tgt, e->adj_ck, n, e->partials, e->stream);
     HIP_TRY(hipGetLastError());
     std::vector<double> h(4 * (size_t)nb);
@@ -1633,38 +1693,59 @@ int adjoint_backward_t(gpe_engine_s* e, double* grad, bool device_out = false) {
     const size_t n = e->n, cs = sizeof(cplx<T>);
     const int nt = e->adj_nt, C = e->adj_C;
     const int nck = (nt + C - 1) / C;
-    const unsigned it_end = e->it;
+    const bool stored = e->adj_phi_len >= (size_t)C * n;
+    const PassArgs<T> fwd = base_args<T>(e);
+    PassArgs<T> rev = fwd;  // conj K
+    const cplx<double>* Kc = (const cplx<double>*)e->adj_Ktab;
+    rev.Kx = Kc;
+    rev.Ky = Kc + e->nx;
+    rev.Kz = Kc + e->nx + e->ny;
+    if constexpr (sizeof(T) == 4) {
+        rev.kx_hl = (const cplx<float>*)e->adj_Khl;
+        rev.kyz_hl = (const cplx<float>*)e->adj_Khl + 2 * e->nx;
+    }
+    // psi is the work array of the recomputed steps until the end
     HIP_TRY(hipMemcpyAsync(e->adj_fin, e->A, n * cs, hipMemcpyDeviceToDevice, e->stream));
     launch_adjoint_lam_init<T>(e->adj_lam, e->adj_tgt, e->adj_fr, e->adj_fi, n, e->stream);
     HIP_TRY(hipMemsetAsync(e->adj_grad, 0, n * sizeof(double), e->stream));
-    AdjArgs a = adj_args<T>(e);
+    AdjArgs<T> a = adj_args<T>(e);
+    cplx<T>*seg = (cplx<T>*)e->adj_seg, *phi = (cplx<T>*)e->adj_phi;
     for (int sg = nck - 1; sg >= 0; sg--) {
-        const int k0 = sg * C, k1 = std::min(nt, k0 + C);
-        char* seg = (char*)e->adj_seg;
-        HIP_TRY(hipMemcpyAsync(e->A, (char*)e->adj_ck + (size_t)sg * n * cs, n * cs, hipMemcpyDeviceToDevice,
-                               e->stream));
-        HIP_TRY(hipMemcpyAsync(seg, e->A, n * cs, hipMemcpyDeviceToDevice, e->stream));
-        e->it = e->adj_it0 + (unsigned)k0;
-        for (int j = 1; j <= k1 - k0; j++) {
-            int r = evolve_t<T>(e, 1, nullptr, 0, false);
-            if (r) return r;
-            HIP_TRY(hipMemcpyAsync(seg + (size_t)j * n * cs, e->A, n * cs, hipMemcpyDeviceToDevice, e->stream));
-        }
-        for (int k = k1 - 1; k >= k0; k--) {
-            a.psi0 = seg + (size_t)(k - k0) * n * cs;
-            a.psi1 = seg + (size_t)(k - k0 + 1) * n * cs;
-            launch_adjoint_step<T>(a, 1, e->stream);
-            kinetic_apply<T>(e, e->adj_phi, false);
-            launch_adjoint_step<T>(a, 2, e->stream);
-            kinetic_apply<T>(e, e->adj_lam, true);
-            launch_adjoint_step<T>(a, 3, e->stream);
-            kinetic_apply<T>(e, e->adj_lam, true);
-            launch_adjoint_step<T>(a, 4, e->stream);
+        const int k0 = sg * C, len = std::min(nt, k0 + C) - k0;
+        HIP_TRY(hipMemcpyAsync(seg, (cplx<T>*)e->adj_ck + (size_t)sg * n, n * cs, hipMemcpyDeviceToDevice, e->stream));
+        adj_steps<T>(
+            e, len, seg, [&](int j) -> void* { return seg + (size_t)(j + 1) * n; },
+            [&](int j) -> void* { return stored ? phi + (size_t)j * n : nullptr; });
+        // the predictor end of step j of the segment
+        auto predictor = [&](int j) -> const cplx<T>* {
+            if (stored) return phi + (size_t)j * n;
+            PassArgs<T> f = fwd;
+            f.psiA = seg + (size_t)j * n;
+            run_pass<T>(e, f, {2, nullptr, e->B, -1, 0, LOAD_PSI0, MID_NONE, STORE_PLAIN, F_VSTEP1, 0});
+            kinetic_kz<T>(e, f, e->B);
+            run_pass<T>(e, f, {2, e->B, phi, 1, 0, LOAD_PLAIN, MID_PART1, STORE_PLAIN, 0, 0});
+            return phi;
+        };
+        a.phi3 = predictor(len - 1);
+        for (int j = len - 1; j >= 0; j--) {
+            a.psi0 = seg + (size_t)j * n;
+            a.psi1 = seg + (size_t)(j + 1) * n;
+            if (j == len - 1) adj_zpass<T>(e, a, ADJ_P2);
+            kinetic_kz<T>(e, rev, a.lam);
+            adj_zpass<T>(e, a, ADJ_P3);
+            kinetic_kz<T>(e, rev, a.lam);
+            if (j > 0) {
+                a.psi0p = seg + (size_t)(j - 1) * n;
+                a.phi3p = predictor(j - 1);
+                adj_zpass<T>(e, a, ADJ_P4P2);
+                a.phi3 = a.phi3p;
+            } else {
+                adj_zpass<T>(e, a, ADJ_P4);
+            }
         }
         HIP_TRY(hipGetLastError());
     }
     HIP_TRY(hipMemcpyAsync(e->A, e->adj_fin, n * cs, hipMemcpyDeviceToDevice, e->stream));
-    e->it = it_end;
     HIP_TRY(hipMemcpyAsync(grad, e->adj_grad, n * sizeof(double),
                            device_out ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));

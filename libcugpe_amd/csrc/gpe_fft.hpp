@@ -439,7 +439,6 @@ enum MidMode {
     MID_KIN_SUM = 7,     // sum |k|^2 |psi_k|^2 (kinetic energy by Parseval)
     MID_KA = 8,          // k_a / (gamma N) (orginal 1125-1162)
     MID_OVERLAP_RE = 9,  // Re(conj psi * v) -> real output (orginal 1067-1074)
-    MID_EXPTC = 10,      // conj(Kx Ky Kz)/N: the adjoint of the kinetic factor
     MID_VPP = 11,        // Vpp(k)/N: dipolar convolution kernel (dev/gpe_engine.cu:960-975)
     MID_VPP_SUM = 12,    // sum Vpp(k) |rho_k|^2 (dev/gpe_engine.cu:1716-1735)
     // the kinetic factor split by axis, K = (K_y K_z) K_x: K_y K_z in a y
@@ -448,6 +447,7 @@ enum MidMode {
     MID_DIP_STEP = 14,   // psi exp(c (Vext + Vdip)), Vdip the real part of the value (dev/gpe_engine.cu:984-1008)
     MID_DIP_RHO = 15,    // psi stored, its density goes on (dev/gpe_engine.cu:618-626)
     MID_DIP_E2 = 16,     // sum rho Vdip (dev/gpe_engine.cu:1768-1782)
+    MID_VSTEP2P = 17,    // MID_VSTEP2 that also stores phi3 (the adjoint's recomputed steps)
 };
 
 // Fourier transform of the particle-particle potential of z-polarised dipoles
@@ -491,6 +491,7 @@ struct PassArgs {
     const cplx<T>* twlo;   // complex64: exp(-2 pi i m / N) - tw, the low part
     cplx<T>* psiA;         // the wave function buffer (psi0 / psi1)
     T* vbuf;               // corrector potential V1 per point
+    cplx<T>* phi3;         // predictor end per point (MID_VSTEP2P)
     T* vq;                 // quantum-friction potential per point
     double* rout;          // real FP64 output (currents)
     const cplx<double>* Kx;  // kinetic factors in FP64, Kz includes 1/N
@@ -624,14 +625,14 @@ __device__ __forceinline__ cplx<T> apply_pin(const PassArgs<T>& a, cplx<T> v, co
 __device__ __forceinline__ double dens64(double g, double x, double y) { return g * (x * x + y * y); }
 
 // k-space factors of the lean passes, one per compile-time kind; MK_EXPT_HL is
-// the complex64 x-axis form of MID_EXPT / MID_EXPTC with the compensated
+// the complex64 x-axis form of MID_EXPT with the compensated
 // tables, MK_EXPT_64 the FP64 product, MK_SEP the per-axis factor of
 // MID_EXPT_SEP (AX: the pass axis, -1 when only known at run time)
 enum MidKind { MK_EXPT_64 = 0, MK_EXPT_HL = 1, MK_K2 = 2, MK_VPP = 3, MK_KA = 4, MK_SEP = 5 };
 
 // kx: the pass's factor staged in LDS, or null: complex64 the x pass's K_x
 // pairs (hi.x, hi.y, lo.x, lo.y), complex128 K_x (x pass) or K_y (y pass)
-template <int MK, bool CJ, typename T, int AX = -1>
+template <int MK, typename T, int AX = -1>
 __device__ __forceinline__ cplx<T> mid_op_lean_k(const PassArgs<T>& a, const Coord& c, cplx<T> v,
                                                  const float4* kx = nullptr) {
     if constexpr (MK == MK_SEP) {
@@ -667,13 +668,11 @@ __device__ __forceinline__ cplx<T> mid_op_lean_k(const PassArgs<T>& a, const Coo
         const unsigned yz = c.iy * (unsigned)a.ph.nz + c.iz;
         cplx<float> h1 = a.kx_hl[2 * c.ix], l1 = a.kx_hl[2 * c.ix + 1];
         cplx<float> h2 = a.kyz_hl[2 * yz], l2 = a.kyz_hl[2 * yz + 1];
-        if (CJ) { h1.y = -h1.y; l1.y = -l1.y; h2.y = -h2.y; l2.y = -l2.y; }
         v = cmul_comp(v, h1, l1);
         return cmul_comp(v, h2, l2);
     } else if constexpr (MK == MK_EXPT_64 || MK == MK_EXPT_HL) {
         cplx<double> w = mk((double)v.x, (double)v.y);
         cplx<double> kx = a.Kx[c.ix], ky = a.Ky[c.iy], kz = a.Kz[c.iz];
-        if (CJ) { kx.y = -kx.y; ky.y = -ky.y; kz.y = -kz.y; }
         w = cmul(w, kx);
         w = cmul(w, ky);
         w = cmul(w, kz);
@@ -691,13 +690,11 @@ __device__ __forceinline__ cplx<T> mid_op_lean_k(const PassArgs<T>& a, const Coo
     }
 }
 
-// the kind and conjugation of a lean mid op; false when it has none
+// the kind of a lean mid op; false when it has none
 template <typename T>
-__host__ __device__ __forceinline__ bool mid_kind(const PassArgs<T>& a, int& mk, bool& cj) {
-    cj = (a.mid_mode == MID_EXPTC);
+__host__ __device__ __forceinline__ bool mid_kind(const PassArgs<T>& a, int& mk) {
     switch (a.mid_mode) {
     case MID_EXPT:
-    case MID_EXPTC:
         mk = (sizeof(T) == 4 && a.axis == 0 && a.kx_hl) ? MK_EXPT_HL : MK_EXPT_64;
         return true;
     case MID_K2: mk = MK_K2; return true;
@@ -711,15 +708,14 @@ __host__ __device__ __forceinline__ bool mid_kind(const PassArgs<T>& a, int& mk,
 template <typename T>
 __device__ __forceinline__ cplx<T> mid_op_lean(const PassArgs<T>& a, const Coord& c, cplx<T> v) {
     int mk;
-    bool cj;
-    if (!mid_kind(a, mk, cj)) return v;
+    if (!mid_kind(a, mk)) return v;
     switch (mk) {
-    case MK_EXPT_HL: return cj ? mid_op_lean_k<MK_EXPT_HL, true>(a, c, v) : mid_op_lean_k<MK_EXPT_HL, false>(a, c, v);
-    case MK_EXPT_64: return cj ? mid_op_lean_k<MK_EXPT_64, true>(a, c, v) : mid_op_lean_k<MK_EXPT_64, false>(a, c, v);
-    case MK_K2: return mid_op_lean_k<MK_K2, false>(a, c, v);
-    case MK_VPP: return mid_op_lean_k<MK_VPP, false>(a, c, v);
-    case MK_SEP: return mid_op_lean_k<MK_SEP, false>(a, c, v);
-    default: return mid_op_lean_k<MK_KA, false>(a, c, v);
+    case MK_EXPT_HL: return mid_op_lean_k<MK_EXPT_HL>(a, c, v);
+    case MK_EXPT_64: return mid_op_lean_k<MK_EXPT_64>(a, c, v);
+    case MK_K2: return mid_op_lean_k<MK_K2>(a, c, v);
+    case MK_VPP: return mid_op_lean_k<MK_VPP>(a, c, v);
+    case MK_SEP: return mid_op_lean_k<MK_SEP>(a, c, v);
+    default: return mid_op_lean_k<MK_KA>(a, c, v);
     }
 }
 
@@ -808,11 +804,12 @@ template <int MM, bool UH = false, typename T>
 __device__ __forceinline__ cplx<T> mid_op_m(const PassArgs<T>& a, const ElemIn<T>& e, cplx<T> v, double* acc) {
     const bool qf = (a.flags & F_QF) != 0;
     const unsigned off = e.c.off;
-    if constexpr (MM == MID_VSTEP2) {
+    if constexpr (MM == MID_VSTEP2 || MM == MID_VSTEP2P) {
         // orginal/gpe_engine.cu:774-801 (and the _part1/_part2[_qf] pair for qf)
         const cplx<T> psi0 = modify_at<UH>(a, e, e.aux, e.it);
         const T V0 = pot2<UH>(a, e.vx, psi0, qf, e.raux, e.it, off);
         const cplx<T> phi3 = mul_exp(v, a.ph.c.x * V0, a.ph.c.y * V0);
+        if constexpr (MM == MID_VSTEP2P) a.phi3[off] = phi3;
         T lv;
         const T d1 = dedfdn<UH>(a.ph, density(a.ph, phi3), e.it + 1, off);
         if (qf) lv = (T)0.5 * (V0 + e.vx1 + d1 + e.raux);
@@ -877,7 +874,7 @@ __device__ __forceinline__ cplx<T> mid_op_m(const PassArgs<T>& a, const ElemIn<T
     } else if constexpr (MM == MID_DIP_E2) {
         acc[0] += dens64((double)a.ph.gamma, (double)e.aux.x, (double)e.aux.y) * (double)v.x;
         return v;
-    } else if constexpr (MM == MID_EXPT || MM == MID_EXPTC || MM == MID_K2 || MM == MID_KA || MM == MID_VPP ||
+    } else if constexpr (MM == MID_EXPT || MM == MID_K2 || MM == MID_KA || MM == MID_VPP ||
                          MM == MID_EXPT_SEP) {
         return mid_op_lean(a, e.c, v);
     } else {
@@ -889,6 +886,7 @@ template <bool UH, typename T>
 __device__ __forceinline__ cplx<T> mid_op2(const PassArgs<T>& a, const ElemIn<T>& e, cplx<T> v, double* acc) {
     switch (a.mid_mode) {
     case MID_VSTEP2: return mid_op_m<MID_VSTEP2, UH>(a, e, v, acc);
+    case MID_VSTEP2P: return mid_op_m<MID_VSTEP2P, UH>(a, e, v, acc);
     case MID_PART1: return mid_op_m<MID_PART1, UH>(a, e, v, acc);
     case MID_VSTEP3: return mid_op_m<MID_VSTEP3, UH>(a, e, v, acc);
     case MID_QF_VSTEP1: return mid_op_m<MID_QF_VSTEP1, UH>(a, e, v, acc);
@@ -899,7 +897,6 @@ __device__ __forceinline__ cplx<T> mid_op2(const PassArgs<T>& a, const ElemIn<T>
     case MID_DIP_RHO: return mid_op_m<MID_DIP_RHO, UH>(a, e, v, acc);
     case MID_DIP_E2: return mid_op_m<MID_DIP_E2, UH>(a, e, v, acc);
     case MID_EXPT:
-    case MID_EXPTC:
     case MID_K2:
     case MID_KA:
     case MID_VPP:
@@ -1189,7 +1186,7 @@ __device__ __forceinline__ void load_regs(const PassArgs<T>& a, unsigned p0, cpl
     }
 }
 
-template <int MK, bool CJ, typename T, int N, int W, bool CONTIG, int R, int PER, int AX = -1>
+template <int MK, typename T, int N, int W, bool CONTIG, int R, int PER, int AX = -1>
 __device__ __forceinline__ void mid_regs_k(const PassArgs<T>& a, unsigned p0, cplx<T> (&v)[PER][R],
                                            const float4* kx = nullptr) {
     constexpr int M = N / R;
@@ -1208,7 +1205,7 @@ __device__ __forceinline__ void mid_regs_k(const PassArgs<T>& a, unsigned p0, cp
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 const Coord c = elem<AX>(a, pc, (unsigned)(j + r * M));
-                v[q][r] = mid_op_lean_k<MK, CJ, T, AX>(a, c, v[q][r], kx);
+                v[q][r] = mid_op_lean_k<MK, T, AX>(a, c, v[q][r], kx);
             }
         }
     }
@@ -1246,7 +1243,7 @@ constexpr int lean_w() {
 // What follows the first stage of a lean pass of two or more stages (the first
 // stage's output is in LDS): the remaining stages, the mid op, the optional
 // second transform and the store of tile p0.
-template <typename T, int N, int W, bool CONTIG, int S1, int S2, int MK, bool CJ, int AX, int PV = 0>
+template <typename T, int N, int W, bool CONTIG, int S1, int S2, int MK, int AX, int PV = 0>
 __device__ __forceinline__ void lean_tail(const PassArgs<T>& a, unsigned p0, cplx<T>* lds, const TwE<T>* tw,
                                           const float4* kx = nullptr) {
     constexpr FftPlan P = plan_of(N, false, sizeof(T) == 4, PV);
@@ -1256,7 +1253,7 @@ __device__ __forceinline__ void lean_tail(const PassArgs<T>& a, unsigned p0, cpl
     cplx<T> v[PERL][RL];
     lds_stages<T, N, W, CONTIG, S1, false, 1, NSG - 1, PV>(lds, tw);
     last_stage_regs<T, N, W, CONTIG, S1, RL, PERL>(lds, tw, v);
-    if constexpr (MK >= 0) mid_regs_k<MK, CJ, T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, kx);
+    if constexpr (MK >= 0) mid_regs_k<MK, T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, kx);
     if constexpr (S2 != 0) {
         constexpr FftPlan Q = plan_of(N, true, sizeof(T) == 4, PV);
         static_assert(Q.r[0] == RL, "reversed plan must start with the last radix");
@@ -1293,11 +1290,11 @@ __device__ __forceinline__ unsigned tile_of_block(unsigned b) {
     }
 }
 
-// MK: compile-time kind of the mid op (MidKind), -1 for none; CJ conjugates it
+// MK: compile-time kind of the mid op (MidKind), -1 for none
 // stage(): writes the workgroup's LDS tables (twiddles, factor), called
 // once the tile's first loads are issued; the first barrier after it orders
 // the writes before any use
-template <typename T, int N, bool CONTIG, int S1, int S2, int WD, int MK, bool CJ, int AX, int PV, typename F>
+template <typename T, int N, bool CONTIG, int S1, int S2, int WD, int MK, int AX, int PV, typename F>
 __device__ __forceinline__ void lean_body(const PassArgs<T>& a, cplx<T>* lds, const TwE<T>* tw, const float4* kx,
                                           F&& stage) {
     constexpr int W = lean_w<T, N, WD>();
@@ -1313,7 +1310,7 @@ __device__ __forceinline__ void lean_body(const PassArgs<T>& a, cplx<T>* lds, co
 #pragma unroll
         for (int q = 0; q < PERL; q++) dft<RL, S1>(v[q]);
         if (kx) __syncthreads();  // the LDS factor table is written
-        if constexpr (MK >= 0) mid_regs_k<MK, CJ, T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, kx);
+        if constexpr (MK >= 0) mid_regs_k<MK, T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, kx);
         if constexpr (S2 != 0) {
 #pragma unroll
             for (int q = 0; q < PERL; q++) dft<RL, S2>(v[q]);
@@ -1329,7 +1326,7 @@ __device__ __forceinline__ void lean_body(const PassArgs<T>& a, cplx<T>* lds, co
         first_stage_global_pre<T, N, W, CONTIG, S1, P.r[0], AX>(a, p0, lds, stage);
         if constexpr (!CONTIG) __builtin_amdgcn_s_setprio(0);
         __syncthreads();
-        lean_tail<T, N, W, CONTIG, S1, S2, MK, CJ, AX, PV>(a, p0, lds, tw, kx);
+        lean_tail<T, N, W, CONTIG, S1, S2, MK, AX, PV>(a, p0, lds, tw, kx);
     }
 }
 
@@ -1396,7 +1393,7 @@ __device__ __forceinline__ void first_stage_stage(const cplx<float>* stage, cplx
     }
 }
 
-template <int N, int SHAPE, int MK, bool CJ, int AX>
+template <int N, int SHAPE, int MK, int AX>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void fft_pipe_kernel(const PassArgs<float> a) {
     constexpr int W = lean_w<float, N, 1>();
@@ -1429,7 +1426,7 @@ void fft_pipe_kernel(const PassArgs<float> a) {
         first_stage_stage<N, W, S1, P.r[0]>(stage, lds);
         __syncthreads();  // the staging buffer is free, the tile is in LDS
         if (t + gridDim.x < ntiles) pipe_fetch<N, W, AX>(a, (t + gridDim.x) * (unsigned)W, stage);
-        lean_tail<float, N, W, false, S1, S2, MK, CJ, AX>(a, t * (unsigned)W, lds, tw, KXL ? kxs : nullptr);
+        lean_tail<float, N, W, false, S1, S2, MK, AX>(a, t * (unsigned)W, lds, tw, KXL ? kxs : nullptr);
     }
 }
 
@@ -1473,7 +1470,7 @@ template <typename T>
 __device__ __forceinline__ bool needs_psi0(const PassArgs<T>& a) {
     return a.load_mode == LOAD_PART2 || a.mid_mode == MID_VSTEP2 || a.mid_mode == MID_PART1 ||
            a.mid_mode == MID_QF_VSTEP1 || a.mid_mode == MID_OVERLAP_RE || a.mid_mode == MID_DIP_STEP ||
-           a.mid_mode == MID_DIP_E2;
+           a.mid_mode == MID_DIP_E2 || a.mid_mode == MID_VSTEP2P;
 }
 template <typename T>
 __device__ __forceinline__ const T* real_side(const PassArgs<T>& a) {
@@ -1636,7 +1633,7 @@ __device__ __forceinline__ void full_body(const PassArgs<T>& a, FullLds<T, N, CO
 // 512-point z physics passes of the built-in physics: bounded to 4 waves they
 // need 75-77 VGPRs and no spills (at 2 the compiler spends ~190); with user
 // hooks they would spill, and at 96 and 192 points (wider tiles) too
-template <typename T, int N, bool CONTIG, bool FULL, int SHAPE, int WD = 1, int MK = -1, bool CJ = false, int AX = -1,
+template <typename T, int N, bool CONTIG, bool FULL, int SHAPE, int WD = 1, int MK = -1, int AX = -1,
           bool UH = false, int PV = 0>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : ((FULL && CONTIG && N == 512 && !UH) ? 4 : 2))))
 void fft_pass_kernel(const PassArgs<T> a) {
@@ -1682,10 +1679,10 @@ void fft_pass_kernel(const PassArgs<T> a) {
         // 53.7 us)
         if constexpr (sizeof(T) == 4) {
             stage();
-            lean_body<T, N, CONTIG, S1, S2, WD, MK, CJ, (CONTIG ? 2 : AX), PV>(a, lds, tw, KXL ? kxs : nullptr,
+            lean_body<T, N, CONTIG, S1, S2, WD, MK, (CONTIG ? 2 : AX), PV>(a, lds, tw, KXL ? kxs : nullptr,
                                                                                []() {});
         } else {
-            lean_body<T, N, CONTIG, S1, S2, WD, MK, CJ, (CONTIG ? 2 : AX), PV>(a, lds, tw, KXL ? kxs : nullptr, stage);
+            lean_body<T, N, CONTIG, S1, S2, WD, MK, (CONTIG ? 2 : AX), PV>(a, lds, tw, KXL ? kxs : nullptr, stage);
         }
     } else {
         stage_tw();
@@ -1713,7 +1710,7 @@ void fft_pass_kernel(const PassArgs<T> a) {
 template <typename T>
 inline bool pass_is_lean(const PassArgs<T>& a) {
     return a.load_mode == LOAD_PLAIN && a.flags == 0 && a.nred == 0 &&
-           (a.mid_mode == MID_NONE || a.mid_mode == MID_EXPT || a.mid_mode == MID_EXPTC || a.mid_mode == MID_K2 ||
+           (a.mid_mode == MID_NONE || a.mid_mode == MID_EXPT || a.mid_mode == MID_K2 ||
             a.mid_mode == MID_KA || a.mid_mode == MID_VPP || a.mid_mode == MID_EXPT_SEP);
 }
 

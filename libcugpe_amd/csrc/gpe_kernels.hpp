@@ -6,6 +6,7 @@
 #include "gpe_zwave.hpp"
 #include "gpe_fused.hpp"
 #include "gpe_plane.hpp"
+#include "gpe_adjoint.hpp"
 
 namespace gpe {
 
@@ -30,13 +31,23 @@ unsigned launch_fft_pass(int N, const PassArgs<T>& a, hipStream_t s);
 // the same for one compiled length (one object file per precision and length)
 template <typename T, int N>
 unsigned launch_fft_pass_n(const PassArgs<T>& a, hipStream_t s);
+// one z pass of a backward step of the adjoint (AdjPass of gpe_adjoint.hpp)
+// for z length N; false when that length has no wave split
+template <typename T>
+bool launch_adjoint_z(int N, const AdjArgs<T>& a, int pass, hipStream_t s);
+template <typename T, int N>
+bool launch_adjoint_z_n(const AdjArgs<T>& a, int pass, hipStream_t s);
 
 #define GPE_FFT_LENGTHS(X) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(512)
-#define GPE_DECLARE_PASS(NN)                                                        \
-    template <>                                                                     \
-    unsigned launch_fft_pass_n<float, NN>(const PassArgs<float>& a, hipStream_t s); \
-    template <>                                                                     \
-    unsigned launch_fft_pass_n<double, NN>(const PassArgs<double>& a, hipStream_t s);
+#define GPE_DECLARE_PASS(NN)                                                                  \
+    template <>                                                                               \
+    unsigned launch_fft_pass_n<float, NN>(const PassArgs<float>& a, hipStream_t s);           \
+    template <>                                                                               \
+    unsigned launch_fft_pass_n<double, NN>(const PassArgs<double>& a, hipStream_t s);         \
+    template <>                                                                               \
+    bool launch_adjoint_z_n<float, NN>(const AdjArgs<float>& a, int pass, hipStream_t s);     \
+    template <>                                                                               \
+    bool launch_adjoint_z_n<double, NN>(const AdjArgs<double>& a, int pass, hipStream_t s);
 GPE_FFT_LENGTHS(GPE_DECLARE_PASS)
 #undef GPE_DECLARE_PASS
 
@@ -114,25 +125,10 @@ bool plane_length_ok(int L);
 template <typename T>
 int launch_plane(const PassArgs<T>& a, int L, int mode, unsigned planes, bool uh, hipStream_t s);
 
-// discrete adjoint of the real-time split step (gpe_adjoint.hip)
-struct AdjArgs {
-    int interactions;
-    double gamma;
-    double up[kMaxUserParams];
-    double cx, cy;          // step coefficient c
-    size_t n;
-    const double* vx;       // V_ext per point (FP64)
-    const void* psi0;       // step input and output states
-    const void* psi1;
-    void* phi;              // work: phi1 / phi2 / phi3
-    void* lam;              // adjoint state
-    void* lam0;             // work: the part of the new adjoint state carried to P4
-    double* vb;             // potential sensitivities (FP64)
-    double* grad;           // dL/dV_ext accumulated (FP64)
-};
-// part 1..4: the pointwise kernels P1..P4 of one backward step
+// discrete adjoint of the real-time split step: part P2, P3 or P4 of a
+// backward step as a pointwise kernel (gpe_adjoint.hip)
 template <typename T>
-void launch_adjoint_step(const AdjArgs& a, int part, hipStream_t s);
+void launch_adjoint_point(const AdjArgs<T>& a, int part, hipStream_t s);
 template <typename T>
 void launch_adjoint_vfill(const Phys<T>& ph, double* out, size_t n, hipStream_t s);
 // partials [4][nb]: Re, Im of sum conj(tgt) psi, sum |a0|^2, sum |tgt|^2; nb returned

@@ -18,6 +18,18 @@ unsigned launch_fft_pass_impl(int N, const PassArgs<T>& a, hipStream_t s) {
 #undef GPE_CASE
 }
 
+template <typename T>
+bool launch_adjoint_z_impl(int N, const AdjArgs<T>& a, int pass, hipStream_t s) {
+#define GPE_CASE(NN) \
+    case NN: return launch_adjoint_z_n<T, NN>(a, pass, s);
+    switch (N) {
+        GPE_FFT_LENGTHS(GPE_CASE)
+    default:
+        return false;
+    }
+#undef GPE_CASE
+}
+
 template <typename T, int NN>
 constexpr int min_tile() {
     constexpr int w = full_tile_w<T, NN, true>();
@@ -271,6 +283,10 @@ static inline dim3 ew_grid(unsigned n) { return dim3((n + kThreads - 1) / kThrea
     template <>                                                                                                   \
     unsigned launch_fft_pass<T>(int N, const PassArgs<T>& a, hipStream_t s) {                                     \
         return launch_fft_pass_impl<T>(N, a, s);                                                                  \
+    }                                                                                                             \
+    template <>                                                                                                   \
+    bool launch_adjoint_z<T>(int N, const AdjArgs<T>& a, int pass, hipStream_t s) {                               \
+        return launch_adjoint_z_impl<T>(N, a, pass, s);                                                           \
     }                                                                                                             \
     template <>                                                                                                   \
     int fft_tile_width<T>(int N) {                                                                                \

@@ -31,7 +31,8 @@
 
 namespace gpe {
 
-enum PlaneMode { PL_OPEN = 0, PL_VSTEP2 = 1, PL_VSTEP3_NEXT = 2, PL_VSTEP3_LAST = 3 };
+// PL_VSTEP2P: PL_VSTEP2 that also stores the predictor end phi3
+enum PlaneMode { PL_OPEN = 0, PL_VSTEP2 = 1, PL_VSTEP3_NEXT = 2, PL_VSTEP3_LAST = 3, PL_VSTEP2P = 4 };
 
 // threads of a plane workgroup: 512 for 64 x 64 planes (one butterfly of the
 // last stage per thread), 256 otherwise
@@ -233,6 +234,7 @@ void plane_kernel(const PassArgs<T> a) {
     const T cx = a.ph.c.x, cy = a.ph.c.y;
     double acc[3] = {0.0, 0.0, 0.0};
     cplx<T> v[PER][R];
+    constexpr bool V2 = (MODE == PL_VSTEP2 || MODE == PL_VSTEP2P);
 
     if constexpr (MODE == PL_OPEN) {
         // psi0 with the step's Vstep1 (orginal/gpe_engine.cu:723-772), row-major
@@ -269,8 +271,8 @@ void plane_kernel(const PassArgs<T> a) {
         __syncthreads();
     } else {
         // side inputs of the physics at this thread's last-stage elements, loaded early
-        cplx<T> side_c[MODE == PL_VSTEP2 ? PER : 1][MODE == PL_VSTEP2 ? R : 1];
-        T side_r[MODE == PL_VSTEP2 ? 1 : PER][MODE == PL_VSTEP2 ? 1 : R];
+        cplx<T> side_c[V2 ? PER : 1][V2 ? R : 1];
+        T side_r[V2 ? 1 : PER][V2 ? 1 : R];
 #pragma unroll
         for (int q = 0; q < PER; q++) {
             const int b = threadIdx.x + q * kPlaneThreads;
@@ -279,7 +281,7 @@ void plane_kernel(const PassArgs<T> a) {
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     const unsigned off = base + (unsigned)((j + r * M) * L + w);
-                    if constexpr (MODE == PL_VSTEP2) side_c[q][r] = ld_nt(a.psiA + off);
+                    if constexpr (V2) side_c[q][r] = ld_nt(a.psiA + off);
                     else side_r[q][r] = ld_nt(a.vbuf + off);
                 }
             }
@@ -300,7 +302,7 @@ void plane_kernel(const PassArgs<T> a) {
             const int w = b % L, j = b / L;
             T vx[R], gv[R], lv[R];
             if constexpr (!UH) plane_vext<false, T, R, M>(a, ix, w, j, base, it, sep, vscale, vx);
-            if constexpr (MODE == PL_VSTEP2) {
+            if constexpr (V2) {
                 // predictor end and corrector potential (orginal/gpe_engine.cu:774-801)
                 if constexpr (!UH) {
                     cplx<T> p0[R];
@@ -311,6 +313,10 @@ void plane_kernel(const PassArgs<T> a) {
 #pragma unroll
                     for (int r = 0; r < R; r++) V0[r] = vx[r] + gv[r];
                     mul_exp_chunk(v[q], V0, cx, cy);  // phi3
+                    if constexpr (MODE == PL_VSTEP2P) {
+#pragma unroll
+                        for (int r = 0; r < R; r++) st_nt(a.phi3 + base + (unsigned)((j + r * M) * L + w), v[q][r]);
+                    }
                     dedfdn_chunk(a.ph, v[q], gv);
 #pragma unroll
                     for (int r = 0; r < R; r++) {

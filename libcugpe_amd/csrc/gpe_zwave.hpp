@@ -331,13 +331,13 @@ void zwave_kernel(const PassArgs<T> a) {
     static_assert(NCH * CH == B, "chunks must tile the points of a lane");
     constexpr bool PRE = (LM != LOAD_PLAIN);   // physics before the first transform
     constexpr bool POST = (MM != MID_NONE);    // physics after it
-    constexpr bool NEED_AUX = (LM == LOAD_PART2) || MM == MID_VSTEP2 || MM == MID_PART1 ||
+    constexpr bool NEED_AUX = (LM == LOAD_PART2) || MM == MID_VSTEP2 || MM == MID_VSTEP2P || MM == MID_PART1 ||
                               MM == MID_QF_VSTEP1 || MM == MID_OVERLAP_RE || MM == MID_DIP_STEP ||
                               MM == MID_DIP_E2;
     const T* rs = real_side(a);
     const bool qf = (a.flags & F_QF) != 0;
     // the fast chunk forms: ops without imprint, built-in physics
-    const bool fast = (MM == MID_VSTEP2) || (MM == MID_VSTEP3 && !(a.flags & F_IMPRINT_NEXT)) ||
+    const bool fast = (MM == MID_VSTEP2) || (MM == MID_VSTEP2P) || (MM == MID_VSTEP3 && !(a.flags & F_IMPRINT_NEXT)) ||
                       (LM == LOAD_PSI0 && !(a.flags & F_IMPRINT)) || (LM == LOAD_PART2 && !(a.flags & F_IMPRINT_MID)) ||
                       MM == MID_PART1 || MM == MID_QF_VSTEP1 || LM == LOAD_RHO || MM == MID_DIP_STEP ||
                       MM == MID_DIP_RHO || MM == MID_DIP_E2;
@@ -435,7 +435,7 @@ void zwave_kernel(const PassArgs<T> a) {
                     for (int j = 0; j < CH; j++)
                         acc[0] += dens64((double)a.ph.gamma, (double)ax[slot][j].x, (double)ax[slot][j].y) * (double)u[j].x;
                 }
-            } else if constexpr (MM == MID_VSTEP2) {
+            } else if constexpr (MM == MID_VSTEP2 || MM == MID_VSTEP2P) {
                 // predictor end and corrector potential (orginal/gpe_engine.cu:774-801)
                 cplx<T> p0[CH];
 #pragma unroll
@@ -445,6 +445,12 @@ void zwave_kernel(const PassArgs<T> a) {
 #pragma unroll
                 for (int j = 0; j < CH; j++) V0[j] = vx[j] + gv[j] + (qf ? rx[slot][j] : (T)0);
                 mul_exp_chunk(u, V0, a.ph.c.x, a.ph.c.y);  // phi3
+                if constexpr (MM == MID_VSTEP2P) {
+                    if (ok) {
+#pragma unroll
+                        for (int j = 0; j < CH; j++) st_nt(&a.phi3[off_of(q * CH + j)], u[j]);
+                    }
+                }
                 dedfdn_chunk(a.ph, u, gv);
 #pragma unroll
                 for (int j = 0; j < CH; j++) lv[j] = (T)0.5 * (V0[j] + vx[j] + gv[j] + (qf ? rx[slot][j] : (T)0));
@@ -609,6 +615,7 @@ unsigned launch_zwave(const PassArgs<T>& a, hipStream_t s) {
         GPE_ZW(SHAPE_I, LOAD_PLAIN, MID_VSTEP3)
         GPE_ZW(SHAPE_I, LOAD_PLAIN, MID_OVERLAP_RE)
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_VSTEP2)
+        GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_VSTEP2P)
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_VSTEP3)
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_QF_VSTEP1)
         GPE_ZW(SHAPE_F, LOAD_RHO, MID_NONE)
