@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <complex>
 #include <cstdlib>
@@ -105,6 +106,14 @@ struct gpe_engine_s {
     bool graph_mid_pin = false;
     unsigned graph_gen = 0, gen = 1;
     bool use_graph = false;  // measured: direct launches are faster on one stream
+
+    // runs of a small lattice on one XCD (gpe_xcd.hpp): the queue words of two
+    // launches (null: not such a lattice), which of them is next, the XCD, and
+    // whether imaginary- and real-time runs may take it (cleared by a launcher
+    // variant set by hand; the autotuner decides for real time)
+    unsigned* xcdq = nullptr;
+    unsigned xcd_home = 0;
+    bool xcd_flip = false, xcd_it = true, xcd_rt = true;
 
     // profiling
     int prof_class = -1;
@@ -584,9 +593,79 @@ int fused_run(gpe_engine_s* e, int nt, hipStream_t s) {
     return 0;
 }
 
+// A small lattice's runs of steps in one kernel on one XCD (gpe_xcd.hpp): the
+// engine's own choice, made where no launcher variant was asked for.  The line
+// lies where one lattice alone on the GPU takes the passes' time, us per step
+// on one XCD / in passes: real time complex64 16^3 17.8 / 20.8, 32x32x24 23.2
+// / 32.1, 16x64x32 19.0 / 24.6, 24x48x32 33.1 / 26.6, complex128 16x24x32 22.9
+// / 25.7, 32x24x24 31.1 / 32.8; planes of 32 x 32: complex64 32^3 14.6 / 18.8,
+// complex128 24x32x32 18.0 / 18.6 (planes of 48 x 48, 27.9 / 27.2 and 30.4 /
+// 27.7, keep their passes); imaginary time complex64 32^3 25.3 / 38.4, 32x64x24
+// 48.9 / 47.9, complex128 48x24x16 31.0 / 34.8, 32^3 30.6 / 40.1.  Several
+// engines at once gain more (three 32^3 complex64: 4.9 / 14.9): each takes an
+// XCD of its own, and the host launches once per 256 steps.
+size_t xcd_most(const gpe_engine_s* e) {
+    const bool c64 = e->precision == GPE_PRECISION_C64;
+    if (e->beta != 0.0) return c64 ? 40960 : 32768;
+    return c64 ? 32768 : 24576;
+}
+
+bool xcd_lattice(const gpe_engine_s* e) {
+    return e->batch == 1 && xcd_length(e->nx) && xcd_length(e->ny) && xcd_length(e->nz) && e->n <= 40960 &&
+           !e->uses_hooks && e->interactions != INT_DIPOLAR;
+}
+
+bool xcd_selected(const gpe_engine_s* e, int pin) {
+    if (!e->xcdq || !(e->beta != 0.0 ? e->xcd_it : e->xcd_rt) || e->n > xcd_most(e) || pin != 0 || e->qf != 0.0 || e->use_graph || e->prof_class >= 0)
+        return false;
+    if (plane_selected(e, pin) && e->nz != 32) return false;
+    // a captured launch would be replayed with the queue words of its first run
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(e->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+}
+
+// nt steps, in launches of at most 256 so that no single kernel runs for long
+template <typename T>
+int xcd_run(gpe_engine_s* e, int nt) {
+    XcdArgs<T> g;
+    g.a = base_args<T>(e);
+    g.a.n1 = (unsigned)e->n;
+    g.B = (cplx<T>*)e->B;
+    const cplx<T>** tw[3] = {&g.twx, &g.twy, &g.twz};
+    const cplx<T>** lo[3] = {&g.twlox, &g.twloy, &g.twloz};
+    for (int a = 0; a < 3; a++) {
+        *tw[a] = (const cplx<T>*)e->tw[a];
+        *lo[a] = (const cplx<T>*)e->twlo[a];
+    }
+    // a workgroup for every 512 points, at most one for each CU of the XCD
+    const unsigned xcds = e->cus >= 256 ? 8u : 1u;
+    g.xcd = e->xcd_home % xcds;
+    g.want = std::min((unsigned)e->cus / xcds, (unsigned)((e->n + 511) / 512));
+    constexpr int kChunk = 256;
+    for (int done = 0; done < nt; done += kChunk) {
+        g.nt = std::min(kChunk, nt - done);
+        g.q = e->xcdq + (e->xcd_flip ? kXqWords : 0);
+        g.qnext = e->xcdq + (e->xcd_flip ? 0 : kXqWords);
+        e->xcd_flip = !e->xcd_flip;
+        if (plane_selected(e, 0)) launch_xcd_plane32<T>(g, xcds * g.want, e->stream);
+        else if (!launch_xcd<T>(e->nz, g, e->beta != 0.0, xcds * g.want, e->stream)) return GPE_ERR_ARG;
+    }
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
 template <typename T>
 int evolve_t(gpe_engine_s* e, int nt, double* mu, int pin, bool mid_pin) {
     if (nt <= 0) return 0;
+    if (xcd_selected(e, pin)) {
+        if (int r = xcd_run<T>(e, nt)) return r;
+        e->it = e->it + (unsigned)nt;
+        if (e->beta != 0.0 && mu) {
+            HIP_TRY(hipMemcpyAsync(mu, e->scal + 2, sizeof(double), hipMemcpyDeviceToHost, e->stream));
+            HIP_TRY(hipStreamSynchronize(e->stream));
+        }
+        return 0;
+    }
     if (fused_selected<T>(e, pin)) {
         if (int r = fused_run<T>(e, nt, e->stream)) return r;
         e->it = e->it + (unsigned)nt;
@@ -743,7 +822,7 @@ void free_all(gpe_engine_s* e) {
                     e->twlo[2], e->Ktab, e->ktab, e->Khl, e->vtab,
                     e->k64, e->updev, e->itdev, e->partials, e->scal, e->rout, e->phase, e->wind, e->adj_ck, e->adj_seg,
                     e->adj_lam, e->adj_phi, e->adj_lam0, e->adj_tgt, e->adj_fin, e->adj_vb, e->adj_grad,
-                    e->adj_vx, e->adj_Ktab, e->adj_Khl};
+                    e->adj_vx, e->adj_Ktab, e->adj_Khl, e->xcdq};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& ev : e->prof_ev) {
@@ -852,11 +931,18 @@ int create_impl(gpe_engine_s** out, const gpe_config_t* cfg, double alpha, doubl
     ALLOC(e->scal, 16 * sizeof(double));
     ALLOC(e->updev, batch * kMaxUserParams * sizeof(double));
     ALLOC(e->itdev, 64);
+    if (xcd_lattice(e)) {
+        // the engines of a process take the XCDs in turn
+        static std::atomic<unsigned> serial{0};
+        e->xcd_home = serial.fetch_add(1);
+        ALLOC(e->xcdq, 2 * kXqWords * sizeof(unsigned));
+    }
 #undef ALLOC
     (void)hipMemset(e->A, 0, nb * 2 * es);
     (void)hipMemset(e->scal, 0, 16 * sizeof(double));
     (void)hipMemset(e->updev, 0, batch * kMaxUserParams * sizeof(double));
     (void)hipMemset(e->itdev, 0, 64);
+    if (e->xcdq) (void)hipMemset(e->xcdq, 0, 2 * kXqWords * sizeof(unsigned));
     int r = (e->precision == GPE_PRECISION_C64) ? upload_static_tables<float>(e) : upload_static_tables<double>(e);
     if (!r) r = upload_potential_any(e);
     if (r) return fail(r);
@@ -2005,8 +2091,29 @@ int autotune_t(gpe_engine_s* e, int steps, int* chosen) {
             const hipError_t h = hipEventSynchronize(t1);
             float ms = 0.f;
             if (h != hipSuccess) err = (int)h;
-            else if (hipEventElapsedTime(&ms, t0, t1) == hipSuccess && ms < best_ms) best |= kVariantFused;
+            else if (hipEventElapsedTime(&ms, t0, t1) == hipSuccess && ms < best_ms) { best |= kVariantFused; best_ms = ms; }
         }
+    }
+    // a small lattice's real-time run on one XCD, kept where it beats the variant
+    // chosen, whose passes serve the runs it does not cover
+    e->variant = best;
+    e->xcd_it = e->xcd_rt = true;
+    if (!err && e->xcdq) {
+        e->beta = 0.0;
+        bool win = xcd_selected(e, 0);
+        if (win) {
+            err = xcd_run<T>(e, 1);
+            (void)hipEventRecord(t0, e->stream);
+            if (!err) err = xcd_run<T>(e, steps);
+            (void)hipEventRecord(t1, e->stream);
+            float ms = 0.f;
+            const hipError_t h = hipEventSynchronize(t1);
+            if (!err && h != hipSuccess) err = (int)h;
+            win = !err && hipEventElapsedTime(&ms, t0, t1) == hipSuccess && ms < best_ms;
+            if (win) best_ms = ms;
+        }
+        e->beta = beta;
+        e->xcd_rt = win;
     }
     (void)hipMemcpyAsync(e->A, save, bytes, hipMemcpyDeviceToDevice, e->stream);
     (void)hipStreamSynchronize(e->stream);
@@ -2043,6 +2150,7 @@ int gpe_engine_set_variant(gpe_engine_t e, int variant) {
     e->gen++;
     if (variant < 0 || variant > 127) return GPE_ERR_ARG;
     e->variant = variant;
+    e->xcd_it = e->xcd_rt = false;
     return 0;
 }
 

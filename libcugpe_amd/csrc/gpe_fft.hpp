@@ -370,12 +370,11 @@ __device__ __forceinline__ void dft(cplx<T>* v) {
 // (w, j + r N/R), applies w_N^(r (j mod NS) N/(NS R)), transforms, and writes
 // (w, (j/NS) NS R + j mod NS + r NS).
 template <typename T, int N, int W, bool CONTIG, int S, int R, int NS>
-__device__ __forceinline__ void fft_stage(cplx<T>* lds, const TwE<T>* tw) {
+__device__ __forceinline__ void fft_stage(cplx<T>* lds, const TwE<T>* tw, const int tid = threadIdx.x) {
     constexpr int NB = W * N / R;
     constexpr int PER = (NB + kThreads - 1) / kThreads;
     constexpr int M = N / R;
     constexpr int TSTEP = N / (NS * R);
-    const int tid = threadIdx.x;
     cplx<T> v[PER][R];
 #pragma unroll
     for (int q = 0; q < PER; q++) {
@@ -604,6 +603,28 @@ __device__ __forceinline__ void st_nt(T* p, T v) {
 template <typename T>
 __device__ __forceinline__ T ld_nt(const T* p) {
     return __builtin_nontemporal_load(p);
+}
+
+// A load that another CU of the same XCD may just have stored to: agent scope,
+// so it is served by the L2 and never by a stale line of this CU's L1 (the
+// runs of gpe_xcd.hpp; an L1 invalidation by an agent acquire fence cost 7 us
+// per barrier there).
+__device__ __forceinline__ float ld_l2(const float* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double ld_l2(const double* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ cplx<float> ld_l2(const cplx<float>* p) {
+    const unsigned long long u =
+        __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return mk(__uint_as_float((unsigned)u), __uint_as_float((unsigned)(u >> 32)));
+}
+__device__ __forceinline__ cplx<double> ld_l2(const cplx<double>* p) { return mk(ld_l2(&p->x), ld_l2(&p->y)); }
+template <bool L2, typename V>
+__device__ __forceinline__ V ld_src(const V* p) {
+    if constexpr (L2) return ld_l2(p);
+    else return *p;
 }
 
 // Phase pinning of the ITE variants: __gpe_imprint_vortexline_zdir_ (dev/gpe_engine.cu:485-511),
@@ -966,10 +987,21 @@ constexpr bool same_plan(const FftPlan& a, const FftPlan& b) {
 // whether a length has an alternative schedule
 constexpr bool has_alt_plan(int N, bool c64) { return !same_plan(alt_plan(N, c64), make_plan(N, c64)); }
 
-// plan of a transform: PV 0 the default schedule, 1 the alternative; rev
+// Radices of four and below: four points per thread, for tiles so few that a
+// workgroup's own chain of instructions is what takes the time (gpe_xcd.hpp)
+constexpr FftPlan fine_plan(int N) {
+    FftPlan p{0, {0, 0, 0, 0, 0, 0, 0, 0}};
+    int n = N;
+    while (n % 4 == 0) { p.r[p.ns++] = 4; n /= 4; }
+    while (n % 3 == 0) { p.r[p.ns++] = 3; n /= 3; }
+    while (n % 2 == 0) { p.r[p.ns++] = 2; n /= 2; }
+    return p;
+}
+
+// plan of a transform: PV 0 the default schedule, 1 the alternative, 2 the fine one; rev
 // reverses the radix order (the second transform of a turn-around pass)
 constexpr FftPlan plan_of(int N, bool rev, bool c64, int pv = 0) {
-    FftPlan p = pv ? alt_plan(N, c64) : make_plan(N, c64);
+    FftPlan p = pv == 2 ? fine_plan(N) : pv ? alt_plan(N, c64) : make_plan(N, c64);
     if (rev)
         for (int i = 0; i < p.ns / 2; i++) {
             int t = p.r[i];
@@ -1077,14 +1109,15 @@ __device__ __forceinline__ void first_stage_global(const PassArgs<T>& a, unsigne
 // first stage of a lean pass from HBM into the LDS tile, calling pre() once
 // after the first loads are issued (the workgroup's table staging then runs
 // while the tile's rows are in flight)
-template <typename T, int N, int W, bool CONTIG, int S, int R, int AX, typename F>
-__device__ __forceinline__ void first_stage_global_pre(const PassArgs<T>& a, unsigned p0, cplx<T>* lds, F&& pre) {
+template <typename T, int N, int W, bool CONTIG, int S, int R, int AX, bool L2, typename F>
+__device__ __forceinline__ void first_stage_global_pre(const PassArgs<T>& a, unsigned p0, cplx<T>* lds, F&& pre,
+                                                       const int tid) {
     constexpr int M = N / R;
     constexpr int NB = W * M;
     constexpr int PER = (NB + kThreads - 1) / kThreads;
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kThreads;
+        const int b = tid + q * kThreads;
         int w = 0, j = 0;
         cplx<T> v[R];
         const bool in = (NB % kThreads) == 0 || b < NB;
@@ -1096,7 +1129,7 @@ __device__ __forceinline__ void first_stage_global_pre(const PassArgs<T>& a, uns
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     const Coord c = elem<AX>(a, pc, (unsigned)(j + r * M));
-                    v[r] = a.src[c.off];
+                    v[r] = ld_src<L2>(&a.src[c.off]);
                 }
             } else {
 #pragma unroll
@@ -1114,12 +1147,12 @@ __device__ __forceinline__ void first_stage_global_pre(const PassArgs<T>& a, uns
 
 // first stage from registers already holding (w, j + r N/R) into LDS
 template <typename T, int N, int W, bool CONTIG, int S, int R, int PER>
-__device__ __forceinline__ void first_stage_regs(cplx<T> (&v)[PER][R], cplx<T>* lds) {
+__device__ __forceinline__ void first_stage_regs(cplx<T> (&v)[PER][R], cplx<T>* lds, const int tid) {
     constexpr int M = N / R;
     constexpr int NB = W * M;
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kThreads;
+        const int b = tid + q * kThreads;
         if ((NB % kThreads) == 0 || b < NB) {
             int w, j;
             bmap<M, W, CONTIG>(b, w, j);
@@ -1132,23 +1165,23 @@ __device__ __forceinline__ void first_stage_regs(cplx<T> (&v)[PER][R], cplx<T>* 
 
 // stages [STAGE, LAST) of plan (N, REV, PV) in LDS
 template <typename T, int N, int W, bool CONTIG, int S, bool REV, int STAGE, int LAST, int PV = 0>
-__device__ __forceinline__ void lds_stages(cplx<T>* lds, const TwE<T>* tw) {
+__device__ __forceinline__ void lds_stages(cplx<T>* lds, const TwE<T>* tw, const int tid = threadIdx.x) {
     if constexpr (STAGE < LAST) {
         constexpr FftPlan P = plan_of(N, REV, sizeof(T) == 4, PV);
-        fft_stage<T, N, W, CONTIG, S, P.r[STAGE], plan_span(P, STAGE)>(lds, tw);
-        lds_stages<T, N, W, CONTIG, S, REV, STAGE + 1, LAST, PV>(lds, tw);
+        fft_stage<T, N, W, CONTIG, S, P.r[STAGE], plan_span(P, STAGE)>(lds, tw, tid);
+        lds_stages<T, N, W, CONTIG, S, REV, STAGE + 1, LAST, PV>(lds, tw, tid);
     }
 }
 
 // last stage (span N/R) from LDS into registers: v[q][r] is element (w, j + r N/R)
 template <typename T, int N, int W, bool CONTIG, int S, int R, int PER>
 __device__ __forceinline__ void last_stage_regs(const cplx<T>* lds, const TwE<T>* tw,
-                                                cplx<T> (&v)[PER][R]) {
+                                                cplx<T> (&v)[PER][R], const int tid = threadIdx.x) {
     constexpr int M = N / R;
     constexpr int NB = W * M;
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kThreads;
+        const int b = tid + q * kThreads;
         if ((NB % kThreads) == 0 || b < NB) {
             int w, j;
             bmap<M, W, CONTIG>(b, w, j);
@@ -1162,13 +1195,13 @@ __device__ __forceinline__ void last_stage_regs(const cplx<T>* lds, const TwE<T>
 }
 
 // registers (w, j + r N/R) <- global memory with the load op (single-stage lengths)
-template <typename T, int N, int W, bool CONTIG, bool FULL, int R, int PER, int AX = -1>
-__device__ __forceinline__ void load_regs(const PassArgs<T>& a, unsigned p0, cplx<T> (&v)[PER][R], double* acc) {
+template <typename T, int N, int W, bool CONTIG, bool L2, int R, int PER, int AX = -1>
+__device__ __forceinline__ void load_regs(const PassArgs<T>& a, unsigned p0, cplx<T> (&v)[PER][R], const int tid) {
     constexpr int M = N / R;
     constexpr int NB = W * M;
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kThreads;
+        const int b = tid + q * kThreads;
         int w, j;
         bmap<M, W, CONTIG>(b, w, j);
         const unsigned p = p0 + (unsigned)w;
@@ -1178,7 +1211,7 @@ __device__ __forceinline__ void load_regs(const PassArgs<T>& a, unsigned p0, cpl
         for (int r = 0; r < R; r++) {
             if (ok) {
                 const Coord c = elem<AX>(a, pc, (unsigned)(j + r * M));
-                v[q][r] = a.src[c.off];
+                v[q][r] = ld_src<L2>(&a.src[c.off]);
             } else {
                 v[q][r] = mk((T)0, (T)0);
             }
@@ -1187,8 +1220,8 @@ __device__ __forceinline__ void load_regs(const PassArgs<T>& a, unsigned p0, cpl
 }
 
 template <int MK, typename T, int N, int W, bool CONTIG, int R, int PER, int AX = -1>
-__device__ __forceinline__ void mid_regs_k(const PassArgs<T>& a, unsigned p0, cplx<T> (&v)[PER][R],
-                                           const float4* kx = nullptr) {
+__device__ __forceinline__ void mid_regs_k(const PassArgs<T>& a, unsigned p0, cplx<T> (&v)[PER][R], const float4* kx,
+                                           const int tid) {
     constexpr int M = N / R;
     constexpr int NB = W * M;
     // keep the factor-table loads here: hoisted above the first transform they
@@ -1196,7 +1229,7 @@ __device__ __forceinline__ void mid_regs_k(const PassArgs<T>& a, unsigned p0, cp
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kThreads;
+        const int b = tid + q * kThreads;
         int w, j;
         bmap<M, W, CONTIG>(b, w, j);
         const unsigned p = p0 + (unsigned)w;
@@ -1212,12 +1245,13 @@ __device__ __forceinline__ void mid_regs_k(const PassArgs<T>& a, unsigned p0, cp
 }
 
 template <typename T, int N, int W, bool CONTIG, int R, int PER, int AX = -1>
-__device__ __forceinline__ void store_regs(const PassArgs<T>& a, unsigned p0, const cplx<T> (&v)[PER][R]) {
+__device__ __forceinline__ void store_regs(const PassArgs<T>& a, unsigned p0, const cplx<T> (&v)[PER][R],
+                                           const int tid = threadIdx.x) {
     constexpr int M = N / R;
     constexpr int NB = W * M;
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kThreads;
+        const int b = tid + q * kThreads;
         int w, j;
         bmap<M, W, CONTIG>(b, w, j);
         const unsigned p = p0 + (unsigned)w;
@@ -1245,29 +1279,29 @@ constexpr int lean_w() {
 // second transform and the store of tile p0.
 template <typename T, int N, int W, bool CONTIG, int S1, int S2, int MK, int AX, int PV = 0>
 __device__ __forceinline__ void lean_tail(const PassArgs<T>& a, unsigned p0, cplx<T>* lds, const TwE<T>* tw,
-                                          const float4* kx = nullptr) {
+                                          const float4* kx, const int tid) {
     constexpr FftPlan P = plan_of(N, false, sizeof(T) == 4, PV);
     constexpr int NSG = P.ns;
     constexpr int RL = P.r[NSG - 1];
     constexpr int PERL = (W * (N / RL) + kThreads - 1) / kThreads;
     cplx<T> v[PERL][RL];
-    lds_stages<T, N, W, CONTIG, S1, false, 1, NSG - 1, PV>(lds, tw);
-    last_stage_regs<T, N, W, CONTIG, S1, RL, PERL>(lds, tw, v);
-    if constexpr (MK >= 0) mid_regs_k<MK, T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, kx);
+    lds_stages<T, N, W, CONTIG, S1, false, 1, NSG - 1, PV>(lds, tw, tid);
+    last_stage_regs<T, N, W, CONTIG, S1, RL, PERL>(lds, tw, v, tid);
+    if constexpr (MK >= 0) mid_regs_k<MK, T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, kx, tid);
     if constexpr (S2 != 0) {
         constexpr FftPlan Q = plan_of(N, true, sizeof(T) == 4, PV);
         static_assert(Q.r[0] == RL, "reversed plan must start with the last radix");
         constexpr int RF = Q.r[NSG - 1];
         constexpr int PERF = (W * (N / RF) + kThreads - 1) / kThreads;
         __syncthreads();  // the first transform's last-stage reads are done
-        first_stage_regs<T, N, W, CONTIG, S2, RL, PERL>(v, lds);
+        first_stage_regs<T, N, W, CONTIG, S2, RL, PERL>(v, lds, tid);
         __syncthreads();
-        lds_stages<T, N, W, CONTIG, S2, true, 1, NSG - 1, PV>(lds, tw);
+        lds_stages<T, N, W, CONTIG, S2, true, 1, NSG - 1, PV>(lds, tw, tid);
         cplx<T> u[PERF][RF];
-        last_stage_regs<T, N, W, CONTIG, S2, RF, PERF>(lds, tw, u);
-        store_regs<T, N, W, CONTIG, RF, PERF, AX>(a, p0, u);
+        last_stage_regs<T, N, W, CONTIG, S2, RF, PERF>(lds, tw, u, tid);
+        store_regs<T, N, W, CONTIG, RF, PERF, AX>(a, p0, u, tid);
     } else {
-        store_regs<T, N, W, CONTIG, RL, PERL, AX>(a, p0, v);
+        store_regs<T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, tid);
     }
 }
 
@@ -1291,31 +1325,32 @@ __device__ __forceinline__ unsigned tile_of_block(unsigned b) {
 }
 
 // MK: compile-time kind of the mid op (MidKind), -1 for none
+// tile: the tile of W pencils
 // stage(): writes the workgroup's LDS tables (twiddles, factor), called
 // once the tile's first loads are issued; the first barrier after it orders
 // the writes before any use
-template <typename T, int N, bool CONTIG, int S1, int S2, int WD, int MK, int AX, int PV, typename F>
+template <typename T, int N, bool CONTIG, int S1, int S2, int WD, int MK, int AX, int PV, bool L2 = false, typename F>
 __device__ __forceinline__ void lean_body(const PassArgs<T>& a, cplx<T>* lds, const TwE<T>* tw, const float4* kx,
-                                          F&& stage) {
+                                          unsigned tile, F&& stage, const int tid = threadIdx.x) {
     constexpr int W = lean_w<T, N, WD>();
     constexpr FftPlan P = plan_of(N, false, sizeof(T) == 4, PV);
     constexpr int NSG = P.ns;
     constexpr int RL = P.r[NSG - 1];
     constexpr int PERL = (W * (N / RL) + kThreads - 1) / kThreads;
-    const unsigned p0 = tile_of_block<T, W, CONTIG>(blockIdx.x) * (unsigned)W;
+    const unsigned p0 = tile * (unsigned)W;
     if constexpr (NSG == 1) {
         cplx<T> v[PERL][RL];
-        load_regs<T, N, W, CONTIG, false, RL, PERL, AX>(a, p0, v, nullptr);
+        load_regs<T, N, W, CONTIG, L2, RL, PERL, AX>(a, p0, v, tid);
         stage();
 #pragma unroll
         for (int q = 0; q < PERL; q++) dft<RL, S1>(v[q]);
         if (kx) __syncthreads();  // the LDS factor table is written
-        if constexpr (MK >= 0) mid_regs_k<MK, T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, kx);
+        if constexpr (MK >= 0) mid_regs_k<MK, T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, kx, tid);
         if constexpr (S2 != 0) {
 #pragma unroll
             for (int q = 0; q < PERL; q++) dft<RL, S2>(v[q]);
         }
-        store_regs<T, N, W, CONTIG, RL, PERL, AX>(a, p0, v);
+        store_regs<T, N, W, CONTIG, RL, PERL, AX>(a, p0, v, tid);
     } else {
         // strided tiles: the waves issuing a tile's loads (and its first
         // stage) run at raised priority, so their requests go out ahead of
@@ -1323,10 +1358,10 @@ __device__ __forceinline__ void lean_body(const PassArgs<T>& a, cplx<T>* lds, co
         // 51.8 -> 50.8 us, x 50.2 -> 49.5 us; the same in the z-wave passes
         // measured slower)
         if constexpr (!CONTIG) __builtin_amdgcn_s_setprio(3);
-        first_stage_global_pre<T, N, W, CONTIG, S1, P.r[0], AX>(a, p0, lds, stage);
+        first_stage_global_pre<T, N, W, CONTIG, S1, P.r[0], AX, L2>(a, p0, lds, stage, tid);
         if constexpr (!CONTIG) __builtin_amdgcn_s_setprio(0);
         __syncthreads();
-        lean_tail<T, N, W, CONTIG, S1, S2, MK, AX, PV>(a, p0, lds, tw, kx);
+        lean_tail<T, N, W, CONTIG, S1, S2, MK, AX, PV>(a, p0, lds, tw, kx, tid);
     }
 }
 
@@ -1426,7 +1461,7 @@ void fft_pipe_kernel(const PassArgs<float> a) {
         first_stage_stage<N, W, S1, P.r[0]>(stage, lds);
         __syncthreads();  // the staging buffer is free, the tile is in LDS
         if (t + gridDim.x < ntiles) pipe_fetch<N, W, AX>(a, (t + gridDim.x) * (unsigned)W, stage);
-        lean_tail<float, N, W, false, S1, S2, MK, AX>(a, t * (unsigned)W, lds, tw, KXL ? kxs : nullptr);
+        lean_tail<float, N, W, false, S1, S2, MK, AX>(a, t * (unsigned)W, lds, tw, KXL ? kxs : nullptr, (int)threadIdx.x);
     }
 }
 
@@ -1677,12 +1712,13 @@ void fft_pass_kernel(const PassArgs<T> a) {
         // flight (256^3: y pass 105.3 -> 103.5 us, x 95.3 -> 94.2 us);
         // complex64 stages them first (deferred, its y pass measured 50.9 ->
         // 53.7 us)
+        const unsigned tile = tile_of_block<T, W, CONTIG>(blockIdx.x);
         if constexpr (sizeof(T) == 4) {
             stage();
             lean_body<T, N, CONTIG, S1, S2, WD, MK, (CONTIG ? 2 : AX), PV>(a, lds, tw, KXL ? kxs : nullptr,
-                                                                               []() {});
+                                                                               tile, []() {});
         } else {
-            lean_body<T, N, CONTIG, S1, S2, WD, MK, (CONTIG ? 2 : AX), PV>(a, lds, tw, KXL ? kxs : nullptr, stage);
+            lean_body<T, N, CONTIG, S1, S2, WD, MK, (CONTIG ? 2 : AX), PV>(a, lds, tw, KXL ? kxs : nullptr, tile, stage);
         }
     } else {
         stage_tw();

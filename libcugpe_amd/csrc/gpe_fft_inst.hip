@@ -167,6 +167,10 @@ unsigned launch_fft_pass_n<GPE_REAL, GPE_FFT_N>(const PassArgs<GPE_REAL>& a, hip
     return launch_fft_pass_n_impl<GPE_REAL, GPE_FFT_N>(a, s);
 }
 template <>
+bool launch_xcd_n<GPE_REAL, GPE_FFT_N>(const XcdArgs<GPE_REAL>& g, bool ite, unsigned blocks, hipStream_t s) {
+    return launch_xcd_len<GPE_REAL, GPE_FFT_N>(g, ite, blocks, s);
+}
+template <>
 bool launch_adjoint_z_n<GPE_REAL, GPE_FFT_N>(const AdjArgs<GPE_REAL>& a, int pass, hipStream_t s) {
     return launch_adj_zwave<GPE_REAL, GPE_FFT_N>(a, pass, s);
 }

@@ -7,6 +7,7 @@
 #include "gpe_fused.hpp"
 #include "gpe_plane.hpp"
 #include "gpe_adjoint.hpp"
+#include "gpe_xcd.hpp"
 
 namespace gpe {
 
@@ -37,6 +38,15 @@ template <typename T>
 bool launch_adjoint_z(int N, const AdjArgs<T>& a, int pass, hipStream_t s);
 template <typename T, int N>
 bool launch_adjoint_z_n(const AdjArgs<T>& a, int pass, hipStream_t s);
+// nt steps of a small lattice of z length N on one XCD (gpe_xcd.hpp); false
+// when there is no kernel for the length
+template <typename T>
+bool launch_xcd(int N, const XcdArgs<T>& g, bool ite, unsigned blocks, hipStream_t s);
+template <typename T, int N>
+bool launch_xcd_n(const XcdArgs<T>& g, bool ite, unsigned blocks, hipStream_t s);
+// the same in real time on y-z planes of 32 x 32 points
+template <typename T>
+void launch_xcd_plane32(const XcdArgs<T>& g, unsigned blocks, hipStream_t s);
 
 #define GPE_FFT_LENGTHS(X) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(512)
 #define GPE_DECLARE_PASS(NN)                                                                  \
@@ -47,7 +57,11 @@ bool launch_adjoint_z_n(const AdjArgs<T>& a, int pass, hipStream_t s);
     template <>                                                                               \
     bool launch_adjoint_z_n<float, NN>(const AdjArgs<float>& a, int pass, hipStream_t s);     \
     template <>                                                                               \
-    bool launch_adjoint_z_n<double, NN>(const AdjArgs<double>& a, int pass, hipStream_t s);
+    bool launch_adjoint_z_n<double, NN>(const AdjArgs<double>& a, int pass, hipStream_t s);   \
+    template <>                                                                               \
+    bool launch_xcd_n<float, NN>(const XcdArgs<float>& g, bool ite, unsigned blocks, hipStream_t s);   \
+    template <>                                                                               \
+    bool launch_xcd_n<double, NN>(const XcdArgs<double>& g, bool ite, unsigned blocks, hipStream_t s);
 GPE_FFT_LENGTHS(GPE_DECLARE_PASS)
 #undef GPE_DECLARE_PASS
 

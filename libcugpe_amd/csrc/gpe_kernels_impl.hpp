@@ -19,6 +19,18 @@ unsigned launch_fft_pass_impl(int N, const PassArgs<T>& a, hipStream_t s) {
 }
 
 template <typename T>
+bool launch_xcd_impl(int N, const XcdArgs<T>& g, bool ite, unsigned blocks, hipStream_t s) {
+#define GPE_CASE(NN) \
+    case NN: return launch_xcd_n<T, NN>(g, ite, blocks, s);
+    switch (N) {
+        GPE_FFT_LENGTHS(GPE_CASE)
+    default:
+        return false;
+    }
+#undef GPE_CASE
+}
+
+template <typename T>
 bool launch_adjoint_z_impl(int N, const AdjArgs<T>& a, int pass, hipStream_t s) {
 #define GPE_CASE(NN) \
     case NN: return launch_adjoint_z_n<T, NN>(a, pass, s);
@@ -283,6 +295,10 @@ static inline dim3 ew_grid(unsigned n) { return dim3((n + kThreads - 1) / kThrea
     template <>                                                                                                   \
     unsigned launch_fft_pass<T>(int N, const PassArgs<T>& a, hipStream_t s) {                                     \
         return launch_fft_pass_impl<T>(N, a, s);                                                                  \
+    }                                                                                                             \
+    template <>                                                                                                   \
+    bool launch_xcd<T>(int N, const XcdArgs<T>& g, bool ite, unsigned blocks, hipStream_t s) {                    \
+        return launch_xcd_impl<T>(N, g, ite, blocks, s);                                                          \
     }                                                                                                             \
     template <>                                                                                                   \
     bool launch_adjoint_z<T>(int N, const AdjArgs<T>& a, int pass, hipStream_t s) {                               \

@@ -1,5 +1,5 @@
 // Launchers of the y-z plane passes (gpe_plane.hpp) for the plane sizes
-// that fit in one workgroup's LDS.
+// that fit in one workgroup's LDS, and of the runs of 32 x 32 planes on one XCD.
 #include "gpe_kernels.hpp"
 
 namespace gpe {
@@ -40,6 +40,14 @@ int launch_plane_t(const PassArgs<T>& a, int L, int mode, unsigned planes, bool 
 
 bool plane_length_ok(int L) { return L == 32 || L == 48 || L == 64; }
 
+template <>
+void launch_xcd_plane32<float>(const XcdArgs<float>& g, unsigned blocks, hipStream_t s) {
+    hipLaunchKernelGGL((xcd_plane_kernel<float, 32>), dim3(blocks), dim3(kThreads), 0, s, g);
+}
+template <>
+void launch_xcd_plane32<double>(const XcdArgs<double>& g, unsigned blocks, hipStream_t s) {
+    hipLaunchKernelGGL((xcd_plane_kernel<double, 32>), dim3(blocks), dim3(kThreads), 0, s, g);
+}
 template <>
 int launch_plane<float>(const PassArgs<float>& a, int L, int mode, unsigned planes, bool uh, hipStream_t s) {
     return launch_plane_t<float>(a, L, mode, planes, uh, s);

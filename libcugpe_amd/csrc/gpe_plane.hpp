@@ -67,7 +67,7 @@ __device__ __forceinline__ cplx<T> plane_kin(const PlaneLds<T, L>& S, unsigned i
 // radix-R Stockham stage (span NS) of L pencils of L points; element i of
 // pencil w sits at w * WS + i * IS
 template <typename T, int L, int WS, int IS, int S, int R, int NS>
-__device__ __forceinline__ void plane_stage(cplx<T>* x, const TwE<T>* tw) {
+__device__ __forceinline__ void plane_stage(cplx<T>* x, const TwE<T>* tw, const int tid) {
     constexpr int kPlaneThreads = plane_threads<L>();
     constexpr int M = L / R;
     constexpr int NB = L * M;
@@ -76,7 +76,7 @@ __device__ __forceinline__ void plane_stage(cplx<T>* x, const TwE<T>* tw) {
     cplx<T> v[PER][R];
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kPlaneThreads;
+        const int b = tid + q * kPlaneThreads;
         if ((NB % kPlaneThreads) == 0 || b < NB) {
             const int w = b % L, j = b / L;
 #pragma unroll
@@ -86,7 +86,7 @@ __device__ __forceinline__ void plane_stage(cplx<T>* x, const TwE<T>* tw) {
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kPlaneThreads;
+        const int b = tid + q * kPlaneThreads;
         if ((NB % kPlaneThreads) == 0 || b < NB) {
             const int w = b % L, j = b / L;
             const int k = j % NS;
@@ -105,11 +105,11 @@ __device__ __forceinline__ void plane_stage(cplx<T>* x, const TwE<T>* tw) {
 
 // stages [STAGE, LAST) of the plan of length L
 template <typename T, int L, int WS, int IS, int S, int STAGE, int LAST>
-__device__ __forceinline__ void plane_stages(cplx<T>* x, const TwE<T>* tw) {
+__device__ __forceinline__ void plane_stages(cplx<T>* x, const TwE<T>* tw, const int tid) {
     constexpr FftPlan P = plan_of(L, false, sizeof(T) == 4);
     if constexpr (STAGE < LAST) {
-        plane_stage<T, L, WS, IS, S, P.r[STAGE], plan_span(P, STAGE)>(x, tw);
-        plane_stages<T, L, WS, IS, S, STAGE + 1, LAST>(x, tw);
+        plane_stage<T, L, WS, IS, S, P.r[STAGE], plan_span(P, STAGE)>(x, tw, tid);
+        plane_stages<T, L, WS, IS, S, STAGE + 1, LAST>(x, tw, tid);
     }
 }
 
@@ -126,17 +126,18 @@ struct PlaneLast {
 
 // Last stage of a y transform (element iy of pencil iz at iz + iy (L + 1))
 // into registers: v[q][r] is element iy = j + r M of pencil iz = w, with
-// (w, j) of butterfly b = threadIdx.x + q * kPlaneThreads; ok[q] marks the
+// (w, j) of butterfly b = tid + q * kPlaneThreads; ok[q] marks the
 // butterflies that exist.  Every thread's LDS reads are done on return.
 template <typename T, int L, int S>
 __device__ __forceinline__ void plane_last_y(const cplx<T>* x, const TwE<T>* tw,
-                                             cplx<T> (&v)[PlaneLast<T, L>::PER][PlaneLast<T, L>::R]) {
+                                             cplx<T> (&v)[PlaneLast<T, L>::PER][PlaneLast<T, L>::R],
+                                             const int tid) {
     using PL = PlaneLast<T, L>;
     constexpr int kPlaneThreads = plane_threads<L>();
     constexpr int R = PL::R, M = PL::M, P = L + 1;
 #pragma unroll
     for (int q = 0; q < PL::PER; q++) {
-        const int b = threadIdx.x + q * kPlaneThreads;
+        const int b = tid + q * kPlaneThreads;
         if ((PL::NB % kPlaneThreads) == 0 || b < PL::NB) {
             const int w = b % L, j = b / L;
 #pragma unroll
@@ -191,23 +192,10 @@ __device__ __forceinline__ void plane_vext(const PassArgs<T>& a, unsigned ix, in
     }
 }
 
-// One plane pass (MODE: PlaneMode) over every plane of the batch: workgroup
-// blockIdx.x takes plane (b, ix) = (blockIdx.x / nx, blockIdx.x % nx).  The
-// physics of the middle runs on the registers of the inverse y transform's
-// last stage, and the kinetic factor and the store on those of the forward y
-// transform's last stage.  UH: the user hook file (per-element ops).
-template <typename T, int L, int MODE, bool UH>
-__global__ __launch_bounds__(plane_threads<L>()) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && L >= 64 ? 4 : 2)))
-void plane_kernel(const PassArgs<T> a) {
-    using PL = PlaneLast<T, L>;
+// the tables of a plane workgroup, before the barrier of the first plane's loads
+template <typename T, int L>
+__device__ __forceinline__ void plane_tables(const PassArgs<T>& a, PlaneLds<T, L>& S) {
     constexpr int kPlaneThreads = plane_threads<L>();
-    constexpr int P = L + 1;
-    constexpr int NPT = L * L;
-    constexpr int PE = NPT / kPlaneThreads;  // elements per thread in the row-major loops
-    static_assert(NPT % kPlaneThreads == 0, "plane size");
-    constexpr int R = PL::R, M = PL::M, PER = PL::PER;
-    constexpr int NS = plan_of(L, false, sizeof(T) == 4).ns;
-    __shared__ PlaneLds<T, L> S;
     for (int i = threadIdx.x; i < L; i += kPlaneThreads) {
         if constexpr (sizeof(T) == 4) {
             const cplx<float> h = a.tw[i], lo = a.twlo[i];
@@ -223,8 +211,23 @@ void plane_kernel(const PassArgs<T> a) {
             S.kz[i].t = a.Kz[i];
         }
     }
+}
+
+// One plane pass (MODE: PlaneMode) on plane pl = (b, ix).  The physics of the
+// middle runs on the registers of the inverse y transform's last stage, and
+// the kinetic factor and the store on those of the forward y transform's last
+// stage.  UH: the user hook file (per-element ops); L2: loads as ld_l2.
+template <typename T, int L, int MODE, bool UH, bool L2>
+__device__ __forceinline__ void plane_tile(const PassArgs<T>& a, PlaneLds<T, L>& S, const unsigned pl, const int tid) {
+    using PL = PlaneLast<T, L>;
+    constexpr int kPlaneThreads = plane_threads<L>();
+    constexpr int P = L + 1;
+    constexpr int NPT = L * L;
+    constexpr int PE = NPT / kPlaneThreads;  // elements per thread in the row-major loops
+    static_assert(NPT % kPlaneThreads == 0, "plane size");
+    constexpr int R = PL::R, M = PL::M, PER = PL::PER;
+    constexpr int NS = plan_of(L, false, sizeof(T) == 4).ns;
     const unsigned nx = (unsigned)a.ph.nx;
-    const unsigned pl = blockIdx.x;
     const unsigned ix = pl % nx;
     const unsigned base = (pl / nx) * a.n1 + ix * (unsigned)NPT;
     const unsigned it = time_index(a.ph);
@@ -234,18 +237,27 @@ void plane_kernel(const PassArgs<T> a) {
     const T cx = a.ph.c.x, cy = a.ph.c.y;
     double acc[3] = {0.0, 0.0, 0.0};
     cplx<T> v[PER][R];
+    // side arrays: non-temporal, from and into this XCD's L2 in the runs of gpe_xcd.hpp
+    auto side_ld = [](const auto* p) __attribute__((always_inline)) {
+        if constexpr (L2) return ld_l2(p);
+        else return ld_nt(p);
+    };
+    auto side_st = [](auto* p, auto w) __attribute__((always_inline)) {
+        if constexpr (L2) *p = w;
+        else st_nt(p, w);
+    };
     constexpr bool V2 = (MODE == PL_VSTEP2 || MODE == PL_VSTEP2P);
 
     if constexpr (MODE == PL_OPEN) {
         // psi0 with the step's Vstep1 (orginal/gpe_engine.cu:723-772), row-major
         cplx<T> u[PE];
 #pragma unroll
-        for (int k = 0; k < PE; k++) u[k] = a.psiA[base + (unsigned)(threadIdx.x + k * kPlaneThreads)];
+        for (int k = 0; k < PE; k++) u[k] = ld_src<L2>(a.psiA + base + (unsigned)(tid + k * kPlaneThreads));
         if constexpr (!UH) {
             T vx[PE], gv[PE];
 #pragma unroll
             for (int k = 0; k < PE; k++) {
-                const int e = threadIdx.x + k * kPlaneThreads;
+                const int e = tid + k * kPlaneThreads;
                 const unsigned iy = (unsigned)(e / L), iz = (unsigned)(e % L);
                 vx[k] = sep ? vscale * (a.ph.vtab[ix] + a.ph.vtab[nx + iy] + a.ph.vtab[nx + a.ph.ny + iz])
                             : vext(a.ph, ix, iy, iz, base + (unsigned)e, it);
@@ -257,7 +269,7 @@ void plane_kernel(const PassArgs<T> a) {
         } else {
 #pragma unroll
             for (int k = 0; k < PE; k++) {
-                const int e = threadIdx.x + k * kPlaneThreads;
+                const int e = tid + k * kPlaneThreads;
                 const unsigned iy = (unsigned)(e / L), iz = (unsigned)(e % L), off = base + (unsigned)e;
                 const ElemIn<T> in = plane_elem<UH>(a, ix, iy, iz, off, it, sep, vscale, false, false);
                 u[k] = load_op_m<LOAD_PSI0, UH>(a, in, u[k], acc);
@@ -265,7 +277,7 @@ void plane_kernel(const PassArgs<T> a) {
         }
 #pragma unroll
         for (int k = 0; k < PE; k++) {
-            const int e = threadIdx.x + k * kPlaneThreads;
+            const int e = tid + k * kPlaneThreads;
             S.x[(e / L) * P + e % L] = u[k];
         }
         __syncthreads();
@@ -275,29 +287,29 @@ void plane_kernel(const PassArgs<T> a) {
         T side_r[V2 ? 1 : PER][V2 ? 1 : R];
 #pragma unroll
         for (int q = 0; q < PER; q++) {
-            const int b = threadIdx.x + q * kPlaneThreads;
+            const int b = tid + q * kPlaneThreads;
             if ((PL::NB % kPlaneThreads) == 0 || b < PL::NB) {
                 const int w = b % L, j = b / L;
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     const unsigned off = base + (unsigned)((j + r * M) * L + w);
-                    if constexpr (V2) side_c[q][r] = ld_nt(a.psiA + off);
-                    else side_r[q][r] = ld_nt(a.vbuf + off);
+                    if constexpr (V2) side_c[q][r] = side_ld(a.psiA + off);
+                    else side_r[q][r] = side_ld(a.vbuf + off);
                 }
             }
         }
 #pragma unroll
         for (int k = 0; k < PE; k++) {
-            const int e = threadIdx.x + k * kPlaneThreads;
-            S.x[(e / L) * P + e % L] = a.src[base + (unsigned)e];
+            const int e = tid + k * kPlaneThreads;
+            S.x[(e / L) * P + e % L] = ld_src<L2>(a.src + base + (unsigned)e);
         }
         __syncthreads();
-        plane_stages<T, L, P, 1, +1, 0, NS>(S.x, S.tw);      // inverse z
-        plane_stages<T, L, 1, P, +1, 0, NS - 1>(S.x, S.tw);  // inverse y but its last stage
-        plane_last_y<T, L, +1>(S.x, S.tw, v);
+        plane_stages<T, L, P, 1, +1, 0, NS>(S.x, S.tw, tid);      // inverse z
+        plane_stages<T, L, 1, P, +1, 0, NS - 1>(S.x, S.tw, tid);  // inverse y but its last stage
+        plane_last_y<T, L, +1>(S.x, S.tw, v, tid);
 #pragma unroll
         for (int q = 0; q < PER; q++) {
-            const int b = threadIdx.x + q * kPlaneThreads;
+            const int b = tid + q * kPlaneThreads;
             if (!((PL::NB % kPlaneThreads) == 0 || b < PL::NB)) continue;
             const int w = b % L, j = b / L;
             T vx[R], gv[R], lv[R];
@@ -315,13 +327,13 @@ void plane_kernel(const PassArgs<T> a) {
                     mul_exp_chunk(v[q], V0, cx, cy);  // phi3
                     if constexpr (MODE == PL_VSTEP2P) {
 #pragma unroll
-                        for (int r = 0; r < R; r++) st_nt(a.phi3 + base + (unsigned)((j + r * M) * L + w), v[q][r]);
+                        for (int r = 0; r < R; r++) side_st(a.phi3 + base + (unsigned)((j + r * M) * L + w), v[q][r]);
                     }
                     dedfdn_chunk(a.ph, v[q], gv);
 #pragma unroll
                     for (int r = 0; r < R; r++) {
                         lv[r] = (T)0.5 * (V0[r] + vx[r] + gv[r]);
-                        st_nt(a.vbuf + base + (unsigned)((j + r * M) * L + w), lv[r]);
+                        side_st(a.vbuf + base + (unsigned)((j + r * M) * L + w), lv[r]);
                     }
                     mul_exp_chunk(p0, lv, cx, cy);
 #pragma unroll
@@ -367,15 +379,15 @@ void plane_kernel(const PassArgs<T> a) {
         if constexpr (MODE == PL_VSTEP3_LAST) return;  // psi1 is in psi (A)
         __syncthreads();
     }
-    plane_stages<T, L, P, 1, -1, 0, NS>(S.x, S.tw);      // forward z
-    plane_stages<T, L, 1, P, -1, 0, NS - 1>(S.x, S.tw);  // forward y but its last stage
-    plane_last_y<T, L, -1>(S.x, S.tw, v);
+    plane_stages<T, L, P, 1, -1, 0, NS>(S.x, S.tw, tid);      // forward z
+    plane_stages<T, L, 1, P, -1, 0, NS - 1>(S.x, S.tw, tid);  // forward y but its last stage
+    plane_last_y<T, L, -1>(S.x, S.tw, v, tid);
     // K_y K_z / N of the split kinetic factor from the LDS tables (per-point
     // loads of a K_y K_z table from global memory had cost a plane pass
     // 11-14%, measured), and the store
 #pragma unroll
     for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kPlaneThreads;
+        const int b = tid + q * kPlaneThreads;
         if ((PL::NB % kPlaneThreads) == 0 || b < PL::NB) {
             const int w = b % L, j = b / L;
 #pragma unroll
@@ -385,6 +397,15 @@ void plane_kernel(const PassArgs<T> a) {
             }
         }
     }
+}
+
+// workgroup blockIdx.x takes plane (b, ix) = (blockIdx.x / nx, blockIdx.x % nx)
+template <typename T, int L, int MODE, bool UH>
+__global__ __launch_bounds__(plane_threads<L>()) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && L >= 64 ? 4 : 2)))
+void plane_kernel(const PassArgs<T> a) {
+    __shared__ PlaneLds<T, L> S;
+    plane_tables<T, L>(a, S);
+    plane_tile<T, L, MODE, UH, false>(a, S, blockIdx.x, (int)threadIdx.x);
 }
 
 }  // namespace gpe

@@ -253,30 +253,37 @@ constexpr int zw_waves() {
     else return phys ? (MM == MID_VSTEP3 ? 4 : ZW_WAVES_PHYS) : 4;
 }
 
-template <typename T, int N, int SHAPE, int LM, int MM>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(zw_waves<T, N, SHAPE, LM, MM>())))
-void zwave_kernel(const PassArgs<T> a) {
-    using Z = ZW<T, N>;
-    constexpr int A = Z::A, B = Z::B;
-    __shared__ ZwLds<T, N> L;
+// stages the twiddles (entry kb A + l) and the z terms of a separable potential
+template <typename T, int N>
+__device__ __forceinline__ void zwave_stage(const PassArgs<T>& a, TwE<T>* tw, T* vzs) {
+    constexpr int A = ZW<T, N>::A;
     const int vk = a.ph.vext;
     const bool sep = (vk == VEXT_HARMONIC || vk == VEXT_COSINE);
     for (int i = threadIdx.x; i < N; i += kThreads) {
         const int m = (i / A) * (i % A);  // row kb = i / A, lane l = i % A
         if constexpr (sizeof(T) == 4) {
             const cplx<float> h = a.tw[m], lo = a.twlo[m];
-            L.tw[i].t = make_float4(h.x, h.y, lo.x, lo.y);
+            tw[i].t = make_float4(h.x, h.y, lo.x, lo.y);
         } else {
-            L.tw[i].t = a.tw[m];
+            tw[i].t = a.tw[m];
         }
-        if (sep) L.vz[i] = a.ph.vtab[a.ph.nx + a.ph.ny + i];
+        if (sep) vzs[i] = a.ph.vtab[a.ph.nx + a.ph.ny + i];
     }
-    __syncthreads();
+}
 
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+// the z pass of one wave, pencils wtask ZW::PW + 0 .. PW - 1 (past the last: none),
+// in a workgroup whose tables are staged; FP64 sums are added to acc; L2: loads as ld_l2
+template <typename T, int N, int SHAPE, int LM, int MM, bool L2 = false>
+__device__ __forceinline__ void zwave_tile(const PassArgs<T>& a, const TwE<T>* tw, const T* vzs, cplx<T>* xs,
+                                           unsigned wtask, double (&acc)[3], const int tid) {
+    using Z = ZW<T, N>;
+    constexpr int A = Z::A, B = Z::B;
+    const int vk = a.ph.vext;
+    const bool sep = (vk == VEXT_HARMONIC || vk == VEXT_COSINE);
+    const int lane = tid & 63, wv = tid >> 6;
     const int g = lane / A, l = lane % A;
-    cplx<T>* X = L.x + wv * Z::WAVE + g * Z::GS;
-    const unsigned p = (blockIdx.x * Z::WAVES + (unsigned)wv) * Z::PW + (unsigned)g;
+    cplx<T>* X = xs + wv * Z::WAVE + g * Z::GS;
+    const unsigned p = wtask * Z::PW + (unsigned)g;
     const bool ok = p < a.M;
     const unsigned pp = ok ? p : 0u;
     const unsigned ny = (unsigned)a.ph.ny, nx = (unsigned)a.ph.nx;
@@ -288,7 +295,12 @@ void zwave_kernel(const PassArgs<T> a) {
     const T vscale = (vk == VEXT_COSINE) ? a.ph.up[0] : (T)1;
     const T vxy = sep ? a.ph.vtab[c.ix] + a.ph.vtab[a.ph.nx + c.iy] : (T)0;
     const unsigned it = time_index(a.ph);
-    double acc[3] = {0.0, 0.0, 0.0};
+    // side arrays: non-temporal, but plain where they stay in this XCD's L2 (there
+    // the non-temporal ones took ~1 us longer to drain before a barrier)
+    auto st = [](auto* p, auto v) __attribute__((always_inline)) {
+        if constexpr (L2) *p = v;
+        else st_nt(p, v);
+    };
     auto off_of = [&](int b) __attribute__((always_inline)) { return base + (unsigned)(A * b); };
 
     // the external potential and the coordinates of register b
@@ -298,7 +310,7 @@ void zwave_kernel(const PassArgs<T> a) {
         e.it = it;
         e.c.iz = (unsigned)(l + A * b);
         e.c.off = base + (unsigned)(A * b);
-        e.vx = sep ? vscale * (vxy + L.vz[l + A * b]) : vext(a.ph, e.c.ix, e.c.iy, e.c.iz, e.c.off, it);
+        e.vx = sep ? vscale * (vxy + vzs[l + A * b]) : vext(a.ph, e.c.ix, e.c.iy, e.c.iz, e.c.off, it);
         e.vx1 = e.vx;
         e.aux = mk((T)0, (T)0);
         e.raux = (T)0;
@@ -310,7 +322,7 @@ void zwave_kernel(const PassArgs<T> a) {
     {
         const cplx<T>* src = (LM == LOAD_PSI0 || LM == LOAD_RHO) ? a.psiA : a.src;
 #pragma unroll
-        for (int b = 0; b < B; b++) v[b] = src[base + (unsigned)(A * b)];
+        for (int b = 0; b < B; b++) v[b] = ld_src<L2>(&src[base + (unsigned)(A * b)]);
     }
 
     // Side inputs (psi0, V1 or V_qf) and the per-point physics run in chunks
@@ -347,11 +359,11 @@ void zwave_kernel(const PassArgs<T> a) {
 #pragma unroll
         for (int j = 0; j < CH; j++) {
             const unsigned off = base + (unsigned)(A * (q * CH + j));
-            ax[slot][j] = NEED_AUX ? ld_nt(&a.psiA[off]) : mk((T)0, (T)0);
+            ax[slot][j] = NEED_AUX ? (L2 ? ld_l2(&a.psiA[off]) : ld_nt(&a.psiA[off])) : mk((T)0, (T)0);
         }
         if (rs) {
 #pragma unroll
-            for (int j = 0; j < CH; j++) rx[slot][j] = ld_nt(&rs[off_of(q * CH + j)]);
+            for (int j = 0; j < CH; j++) rx[slot][j] = L2 ? ld_l2(&rs[off_of(q * CH + j)]) : ld_nt(&rs[off_of(q * CH + j)]);
         } else {
 #pragma unroll
             for (int j = 0; j < CH; j++) rx[slot][j] = (T)0;
@@ -360,7 +372,7 @@ void zwave_kernel(const PassArgs<T> a) {
     auto vx_chunk = [&](int q, T (&vx)[CH]) {
         if (sep) {
 #pragma unroll
-            for (int j = 0; j < CH; j++) vx[j] = vscale * (vxy + L.vz[l + A * (q * CH + j)]);
+            for (int j = 0; j < CH; j++) vx[j] = vscale * (vxy + vzs[l + A * (q * CH + j)]);
         } else {
 #pragma unroll
             for (int j = 0; j < CH; j++) {
@@ -385,7 +397,7 @@ void zwave_kernel(const PassArgs<T> a) {
                     for (int j = 0; j < CH; j++) u[j] = cscale(u[j], f);
                     if (ok) {
 #pragma unroll
-                        for (int j = 0; j < CH; j++) st_nt(&a.psiA[off_of(q * CH + j)], u[j]);
+                        for (int j = 0; j < CH; j++) st(&a.psiA[off_of(q * CH + j)], u[j]);
                     }
                 }
                 if (a.flags & F_VSTEP1) {
@@ -401,7 +413,7 @@ void zwave_kernel(const PassArgs<T> a) {
                     for (int j = 0; j < CH; j++) u[j] = cscale(u[j], f);
                     if (ok) {
 #pragma unroll
-                        for (int j = 0; j < CH; j++) st_nt(&a.psiA[off_of(q * CH + j)], u[j]);
+                        for (int j = 0; j < CH; j++) st(&a.psiA[off_of(q * CH + j)], u[j]);
                     }
                 }
 #pragma unroll
@@ -411,7 +423,7 @@ void zwave_kernel(const PassArgs<T> a) {
                 // the wave function after the kinetic factor, then its density
                 if (ok) {
 #pragma unroll
-                    for (int j = 0; j < CH; j++) st_nt(&a.psiA[off_of(q * CH + j)], u[j]);
+                    for (int j = 0; j < CH; j++) st(&a.psiA[off_of(q * CH + j)], u[j]);
                 }
 #pragma unroll
                 for (int j = 0; j < CH; j++)
@@ -448,7 +460,7 @@ void zwave_kernel(const PassArgs<T> a) {
                 if constexpr (MM == MID_VSTEP2P) {
                     if (ok) {
 #pragma unroll
-                        for (int j = 0; j < CH; j++) st_nt(&a.phi3[off_of(q * CH + j)], u[j]);
+                        for (int j = 0; j < CH; j++) st(&a.phi3[off_of(q * CH + j)], u[j]);
                     }
                 }
                 dedfdn_chunk(a.ph, u, gv);
@@ -456,7 +468,7 @@ void zwave_kernel(const PassArgs<T> a) {
                 for (int j = 0; j < CH; j++) lv[j] = (T)0.5 * (V0[j] + vx[j] + gv[j] + (qf ? rx[slot][j] : (T)0));
                 if (ok) {
 #pragma unroll
-                    for (int j = 0; j < CH; j++) st_nt(&a.vbuf[off_of(q * CH + j)], lv[j]);
+                    for (int j = 0; j < CH; j++) st(&a.vbuf[off_of(q * CH + j)], lv[j]);
                 }
                 mul_exp_chunk(p0, lv, a.ph.c.x, a.ph.c.y);
 #pragma unroll
@@ -480,7 +492,7 @@ void zwave_kernel(const PassArgs<T> a) {
                 for (int j = 0; j < CH; j++) lv[j] = (T)0.5 * (V0[j] + vx[j] + gv[j] + (qf ? rx[slot][j] : (T)0));
                 if (ok) {
 #pragma unroll
-                    for (int j = 0; j < CH; j++) st_nt(&a.vbuf[off_of(q * CH + j)], lv[j]);
+                    for (int j = 0; j < CH; j++) st(&a.vbuf[off_of(q * CH + j)], lv[j]);
                 }
                 mul_exp_chunk(p0, lv, a.ph.c.x, a.ph.c.y);
 #pragma unroll
@@ -508,7 +520,7 @@ void zwave_kernel(const PassArgs<T> a) {
                 for (int j = 0; j < CH; j++) {
                     const T r0 = density(a.ph, p0[j]);
                     const T qv = (p0[j].x * u[j].y + (-p0[j].y) * u[j].x) / (r0 + (T)1.0e-12);
-                    if (ok) st_nt(&a.vq[off_of(q * CH + j)], qv);
+                    if (ok) st(&a.vq[off_of(q * CH + j)], qv);
                     lv[j] = vx[j] + gv[j] + qv;
                 }
                 mul_exp_chunk(p0, lv, a.ph.c.x, a.ph.c.y);
@@ -525,7 +537,7 @@ void zwave_kernel(const PassArgs<T> a) {
                 }
                 if (ok) {
 #pragma unroll
-                    for (int j = 0; j < CH; j++) st_nt(&a.psiA[off_of(q * CH + j)], u[j]);
+                    for (int j = 0; j < CH; j++) st(&a.psiA[off_of(q * CH + j)], u[j]);
                 }
                 if (a.flags & F_NEXT_VSTEP1) {
                     dedfdn_chunk(a.ph, u, gv);
@@ -561,7 +573,7 @@ void zwave_kernel(const PassArgs<T> a) {
             physics(q, q & 1);
         });
     }
-    zw_fft<T, N, S1, B>(v, X, L.tw, l);
+    zw_fft<T, N, S1, B>(v, X, tw, l);
     if constexpr (POST && !EARLY) fetch(0, 0);
     if constexpr (POST) {
         static_for<0, NCH>([&](auto qc) __attribute__((always_inline)) {
@@ -570,12 +582,23 @@ void zwave_kernel(const PassArgs<T> a) {
             physics(q, q & 1);
         });
     }
-    if constexpr (S2 != 0) zw_fft<T, N, S2, B>(v, X, L.tw, l);
+    if constexpr (S2 != 0) zw_fft<T, N, S2, B>(v, X, tw, l);
 
     if (a.store_mode == STORE_PLAIN && ok) {
 #pragma unroll
         for (int b = 0; b < B; b++) a.dst[base + (unsigned)(A * b)] = v[b];
     }
+}
+
+template <typename T, int N, int SHAPE, int LM, int MM>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(zw_waves<T, N, SHAPE, LM, MM>())))
+void zwave_kernel(const PassArgs<T> a) {
+    __shared__ ZwLds<T, N> L;
+    zwave_stage<T, N>(a, L.tw, L.vz);
+    __syncthreads();
+    double acc[3] = {0.0, 0.0, 0.0};
+    zwave_tile<T, N, SHAPE, LM, MM>(a, L.tw, L.vz, L.x, blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6), acc,
+                                    (int)threadIdx.x);
     if (a.nred > 0) {
         const double s0 = block_sum(acc[0], L.red);
         if (threadIdx.x == 0) a.partials[blockIdx.x] = s0;
