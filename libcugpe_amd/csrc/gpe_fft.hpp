@@ -435,7 +435,7 @@ enum MidMode {
     MID_PART1 = 4,       // predictor end only, norm sum (orginal 803-815)
     MID_VSTEP3 = 5,      // corrector end (orginal 870-878), optional next Vstep1
     MID_QF_VSTEP1 = 6,   // QF overlap (orginal 911-922) + Vstep1_qf (orginal 748-772)
-    MID_KIN_SUM = 7,     // sum |k|^2 |psi_k|^2 (kinetic energy by Parseval)
+    MID_KAX_SUM = 7,     // sum k_a^2 |v|^2 along the pass's axis a, nothing stored (kinetic energy by Parseval)
     MID_KA = 8,          // k_a / (gamma N) (orginal 1125-1162)
     MID_OVERLAP_RE = 9,  // Re(conj psi * v) -> real output (orginal 1067-1074)
     MID_VPP = 11,        // Vpp(k)/N: dipolar convolution kernel (dev/gpe_engine.cu:960-975)
@@ -464,7 +464,7 @@ enum PassFlags {
     F_IMPRINT = 2,        // imprint the vortex on the loaded psi0 (written back)
     F_VSTEP1 = 4,         // LOAD_PSI0: apply Vstep1 after the preparation
     F_QF = 8,             // add the stored quantum-friction potential
-    F_RED_POT = 16,       // LOAD_PLAIN: sum rho*Vext and EDF(rho)
+    F_RED_POT = 16,       // LOAD_PLAIN: sum rho*Vext and EDF(rho) (with F_SCALE of the rescaled psi, stored)
     F_RED_NORM = 32,      // sum rho of the produced wave function
     F_NEXT_VSTEP1 = 64,   // MID_VSTEP3: continue with the next step's Vstep1
     F_NEXT_PSI = 128,     // MID_VSTEP3: continue with the next step's psi0 (QF transform)
@@ -774,6 +774,10 @@ __device__ __forceinline__ cplx<T> load_op_m(const PassArgs<T>& a, const ElemIn<
     const unsigned off = e.c.off;
     if constexpr (LM == LOAD_PLAIN) {
         if (a.flags & F_RED_POT) {
+            if (a.flags & F_SCALE) {
+                v = cscale(v, (T)a.scal[1]);
+                a.psiA[off] = v;
+            }
             const double rho = dens64((double)a.ph.gamma, (double)v.x, (double)v.y);
             acc[0] += rho * (double)e.vx;
             acc[1] += edf<UH>(a.ph, a.up64, rho, e.it, off);
@@ -870,10 +874,9 @@ __device__ __forceinline__ cplx<T> mid_op_m(const PassArgs<T>& a, const ElemIn<T
         const cplx<T> m0 = modify_at<UH>(a, e, psi0, e.it);
         const T lv = pot2<UH>(a, e.vx, m0, true, q, e.it, off);
         return mul_exp(m0, a.ph.c.x * lv, a.ph.c.y * lv);
-    } else if constexpr (MM == MID_KIN_SUM) {
-        const double k2 = a.kx64[e.c.ix] * a.kx64[e.c.ix] + a.ky64[e.c.iy] * a.ky64[e.c.iy] +
-                          a.kz64[e.c.iz] * a.kz64[e.c.iz];
-        acc[0] += k2 * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
+    } else if constexpr (MM == MID_KAX_SUM) {
+        // z passes; the strided ones run kax_sum_kernel
+        acc[2] += a.kz64[e.c.iz] * a.kz64[e.c.iz] * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
         return v;
     } else if constexpr (MM == MID_VPP_SUM) {
         const double f = vpp_k(a.up64, a.kx64[e.c.ix], a.ky64[e.c.iy], a.kz64[e.c.iz]);
@@ -911,7 +914,7 @@ __device__ __forceinline__ cplx<T> mid_op2(const PassArgs<T>& a, const ElemIn<T>
     case MID_PART1: return mid_op_m<MID_PART1, UH>(a, e, v, acc);
     case MID_VSTEP3: return mid_op_m<MID_VSTEP3, UH>(a, e, v, acc);
     case MID_QF_VSTEP1: return mid_op_m<MID_QF_VSTEP1, UH>(a, e, v, acc);
-    case MID_KIN_SUM: return mid_op_m<MID_KIN_SUM, UH>(a, e, v, acc);
+    case MID_KAX_SUM: return mid_op_m<MID_KAX_SUM, UH>(a, e, v, acc);
     case MID_VPP_SUM: return mid_op_m<MID_VPP_SUM, UH>(a, e, v, acc);
     case MID_OVERLAP_RE: return mid_op_m<MID_OVERLAP_RE, UH>(a, e, v, acc);
     case MID_DIP_STEP: return mid_op_m<MID_DIP_STEP, UH>(a, e, v, acc);
@@ -1740,6 +1743,62 @@ void fft_pass_kernel(const PassArgs<T> a) {
             if (threadIdx.x == 0) a.partials[2 * (size_t)gridDim.x + blockIdx.x] = s2;
         }
     }
+}
+
+// Forward transform along a strided axis (AX: 0 x, 1 y) and the FP64 sum of
+// k_a^2 |v|^2 over its registers; nothing is written but the workgroup's sum.
+// The kinetic energy needs each axis' transform alone (Parseval along the other
+// two), so its passes read the state once each instead of carrying a 3-D
+// transform through memory: bound by that read.
+template <typename T, int N, int AX>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2)))
+void kax_sum_kernel(const PassArgs<T> a) {
+    constexpr int W = lean_w<T, N, 1>();
+    constexpr FftPlan P = plan_of(N, false, sizeof(T) == 4);
+    constexpr int NSG = P.ns, RL = P.r[NSG - 1], M = N / RL, NB = W * M;
+    constexpr int PERL = (NB + kThreads - 1) / kThreads;
+    __shared__ TwE<T> tw[N];
+    __shared__ cplx<T> lds[lds_elems<T, N, W, false>()];
+    __shared__ double red[kThreads / 64];
+    const int tid = threadIdx.x;
+    const unsigned p0 = blockIdx.x * (unsigned)W;
+    cplx<T> v[PERL][RL];
+    if constexpr (NSG == 1) {
+        load_regs<T, N, W, false, false, RL, PERL, AX>(a, p0, v, tid);
+#pragma unroll
+        for (int q = 0; q < PERL; q++) dft<RL, -1>(v[q]);
+    } else {
+        first_stage_global_pre<T, N, W, false, -1, P.r[0], AX, false>(a, p0, lds, [&]() {
+            for (int i = tid; i < N; i += kThreads) {
+                if constexpr (sizeof(T) == 4) {
+                    const cplx<float> h = a.tw[i], lo = a.twlo[i];
+                    tw[i].t = make_float4(h.x, h.y, lo.x, lo.y);
+                } else {
+                    tw[i].t = a.tw[i];
+                }
+            }
+        }, tid);
+        __syncthreads();
+        lds_stages<T, N, W, false, -1, false, 1, NSG - 1>(lds, tw, tid);
+        last_stage_regs<T, N, W, false, -1, RL, PERL>(lds, tw, v, tid);
+    }
+    const double* k = AX == 0 ? a.kx64 : a.ky64;
+    double acc = 0.0;
+#pragma unroll
+    for (int q = 0; q < PERL; q++) {
+        const int b = tid + q * kThreads;
+        int w, j;
+        bmap<M, W, false>(b, w, j);
+        if (((NB % kThreads) == 0 || b < NB) && p0 + (unsigned)w < a.M) {
+#pragma unroll
+            for (int r = 0; r < RL; r++) {
+                const double kk = k[j + r * M];
+                acc += kk * kk * ((double)v[q][r].x * (double)v[q][r].x + (double)v[q][r].y * (double)v[q][r].y);
+            }
+        }
+    }
+    const double s = block_sum(acc, red);
+    if (tid == 0) a.partials[blockIdx.x] = s;
 }
 
 // the pass can run in the lean kernel

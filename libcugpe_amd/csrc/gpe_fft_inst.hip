@@ -15,6 +15,12 @@ unsigned launch_fft_pass_n_impl(const PassArgs<T>& a, hipStream_t s) {
         const unsigned zb = launch_zwave<T, NN>(a, s);
         if (zb) return zb;
     }
+    if (a.mid_mode == MID_KAX_SUM && a.axis != 2) {
+        const unsigned kb = (a.M + lean_w<T, NN, 1>() - 1) / lean_w<T, NN, 1>();
+        if (a.axis == 0) hipLaunchKernelGGL((kax_sum_kernel<T, NN, 0>), dim3(kb), dim3(kThreads), 0, s, a);
+        else hipLaunchKernelGGL((kax_sum_kernel<T, NN, 1>), dim3(kb), dim3(kThreads), 0, s, a);
+        return kb;
+    }
     // instantiated variants: z lean {F, I}, z full {F, I, IF}, y/x lean {F, I, FI} at full and
     // (variant bit 1) half tile width, y/x full {F}
     const bool lean = pass_is_lean(a);

@@ -73,6 +73,12 @@ enum FinalizeMode {
 void launch_finalize(const double* partials, int nb, int nq, double* scal, int mode, int slot, double npart,
                      double dt, double div, hipStream_t s);
 
+// scal[slot] = V_ext, scal[slot + 1] = interaction and scal[slot + 2] = kinetic
+// energy from the sums of the energy passes: [3][nbz] (potential, EDF, k_z^2),
+// [nby] (k_y^2) and [nbx] (k_x^2), one after another
+void launch_energy_finalize(const double* partials, int nbz, int nby, int nbx, int nx, int ny, int nz, double gamma,
+                            double* scal, int slot, hipStream_t s);
+
 // sum of gamma |psi|^2 over the lattice into partials[0..nb), nb returned
 template <typename T>
 int launch_norm_partials(const cplx<T>* A, unsigned n, double gamma, double* partials, hipStream_t s);

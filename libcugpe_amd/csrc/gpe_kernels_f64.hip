@@ -25,6 +25,32 @@ __global__ __launch_bounds__(kThreads) void finalize_kernel(const double* __rest
 }
 
 
+__global__ __launch_bounds__(kThreads) void energy_finalize_kernel(const double* __restrict__ partials, int nbz, int nby,
+                                                                   int nbx, int nx, int ny, int nz, double gamma,
+                                                                   double* __restrict__ scal, int slot) {
+    __shared__ double red[kThreads / 64];
+    const int nb[5] = {nbz, nbz, nbz, nby, nbx};
+    double sum[5];
+    const double* p = partials;
+    for (int q = 0; q < 5; q++) {
+        double acc = 0.0;
+        for (int b = threadIdx.x; b < nb[q]; b += kThreads) acc += p[b];
+        sum[q] = block_sum(acc, red);
+        p += nb[q];
+    }
+    if (threadIdx.x == 0) {
+        scal[slot] = sum[0];
+        scal[slot + 1] = sum[1];
+        scal[slot + 2] = (sum[2] / nz + sum[3] / ny + sum[4] / nx) / (2.0 * gamma);
+    }
+}
+
+void launch_energy_finalize(const double* partials, int nbz, int nby, int nbx, int nx, int ny, int nz, double gamma,
+                            double* scal, int slot, hipStream_t s) {
+    hipLaunchKernelGGL(energy_finalize_kernel, dim3(1), dim3(kThreads), 0, s, partials, nbz, nby, nbx, nx, ny, nz,
+                       gamma, scal, slot);
+}
+
 bool fft_length_supported(int N) { return fft_tile_width<double>(N) > 0; }
 
 // plain streaming copy (16-byte vectors); reference point for hardware byte counters

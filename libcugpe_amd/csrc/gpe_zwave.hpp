@@ -342,7 +342,7 @@ __device__ __forceinline__ void zwave_tile(const PassArgs<T>& a, const TwE<T>* t
     constexpr int NCH = B / CH;
     static_assert(NCH * CH == B, "chunks must tile the points of a lane");
     constexpr bool PRE = (LM != LOAD_PLAIN);   // physics before the first transform
-    constexpr bool POST = (MM != MID_NONE);    // physics after it
+    constexpr bool POST = (MM != MID_NONE && MM != MID_KAX_SUM);  // physics after it
     constexpr bool NEED_AUX = (LM == LOAD_PART2) || MM == MID_VSTEP2 || MM == MID_VSTEP2P || MM == MID_PART1 ||
                               MM == MID_QF_VSTEP1 || MM == MID_OVERLAP_RE || MM == MID_DIP_STEP ||
                               MM == MID_DIP_E2;
@@ -574,6 +574,15 @@ __device__ __forceinline__ void zwave_tile(const PassArgs<T>& a, const TwE<T>* t
         });
     }
     zw_fft<T, N, S1, B>(v, X, tw, l);
+    if constexpr (MM == MID_KAX_SUM) {
+        if (ok) {
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                const double kk = a.kz64[l + A * b];
+                acc[2] += kk * kk * ((double)v[b].x * (double)v[b].x + (double)v[b].y * (double)v[b].y);
+            }
+        }
+    }
     if constexpr (POST && !EARLY) fetch(0, 0);
     if constexpr (POST) {
         static_for<0, NCH>([&](auto qc) __attribute__((always_inline)) {
@@ -607,6 +616,10 @@ void zwave_kernel(const PassArgs<T> a) {
         const double s1 = block_sum(acc[1], L.red);
         if (threadIdx.x == 0) a.partials[(size_t)gridDim.x + blockIdx.x] = s1;
     }
+    if (a.nred > 2) {
+        const double s2 = block_sum(acc[2], L.red);
+        if (threadIdx.x == 0) a.partials[2 * (size_t)gridDim.x + blockIdx.x] = s2;
+    }
 }
 
 // launches the z pass in the wave kernel when the length and the pass kind
@@ -619,7 +632,7 @@ unsigned launch_zwave(const PassArgs<T>& a, hipStream_t s) {
     } else {
         // engines with user hooks run their z passes in the LDS-tile kernels
         // compiled with the hook file; these kernels carry none of its code
-        if (a.axis != 2 || a.nred > 2 || a.ph.modify) return 0;
+        if (a.axis != 2 || a.nred > 3 || a.ph.modify) return 0;
         const unsigned blocks = (a.M + ZW<T, N>::PENCILS - 1) / ZW<T, N>::PENCILS;
         const int shape = pass_shape(a.dir1, a.dir2);
         const int lm = (a.load_mode == LOAD_PLAIN && (a.flags & F_RED_POT)) ? LOAD_REDPOT : a.load_mode;
@@ -630,7 +643,7 @@ unsigned launch_zwave(const PassArgs<T>& a, hipStream_t s) {
         return blocks;                                                                                \
     }
         GPE_ZW(SHAPE_F, LOAD_PLAIN, MID_NONE)
-        GPE_ZW(SHAPE_F, LOAD_REDPOT, MID_NONE)
+        GPE_ZW(SHAPE_F, LOAD_REDPOT, MID_KAX_SUM)
         GPE_ZW(SHAPE_F, LOAD_PSI0, MID_NONE)
         GPE_ZW(SHAPE_F, LOAD_PART2, MID_NONE)
         GPE_ZW(SHAPE_I, LOAD_PLAIN, MID_NONE)
