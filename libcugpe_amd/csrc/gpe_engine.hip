@@ -1018,9 +1018,9 @@ int cloud_t(gpe_engine_s* e, double epsilon, double* out) {
 
 template <typename T>
 int detect_t(gpe_engine_s* e, double rho_min, int8_t* w, long* count) {
-    if (!e->wind) HIP_TRY(hipMalloc(&e->wind, 3 * e->n));
-    const int nb = launch_windings<T>((const cplx<T>*)e->A, e->nx, e->ny, e->nz, rho_min, e->wind, e->partials,
-                                      e->stream);
+    if (w && !e->wind) HIP_TRY(hipMalloc(&e->wind, 3 * e->n));
+    const int nb = launch_windings<T>((const cplx<T>*)e->A, e->nx, e->ny, e->nz, rho_min, w ? e->wind : nullptr,
+                                      e->partials, e->stream);
     finalize(e, nb, 1, FIN_STORE, kSlotCount, 1.0);
     HIP_TRY(hipGetLastError());
     double c = 0;
