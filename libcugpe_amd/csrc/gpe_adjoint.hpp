@@ -224,7 +224,8 @@ void adj_zwave_kernel(const AdjArgs<T> a) {
 // false: the z length has no wave split
 template <typename T, int N>
 bool launch_adj_zwave(const AdjArgs<T>& a, int pass, hipStream_t s) {
-    if constexpr (zw_lanes<T>(N) == 0) {
+    // (24 points per lane in complex128 leave no registers for the parts)
+    if constexpr (zw_lanes<T>(N) == 0 || (sizeof(T) == 8 && N > 16 * zw_lanes<T>(N))) {
         return false;
     } else {
         const dim3 g((a.M + ZW<T, N>::PENCILS - 1) / ZW<T, N>::PENCILS), b(kThreads);

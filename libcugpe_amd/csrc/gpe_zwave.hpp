@@ -25,7 +25,8 @@
 
 namespace gpe {
 
-// lanes per pencil; 0: the length runs in the LDS-tile kernels.  512 = 16
+// lanes per pencil; 0: the length runs in the LDS-tile kernels (96 and 192 points in
+// complex64 against those, us per step: 96^3 72 -> 69, 128x128x192 129 -> 96, 192^3 268 -> 218).  512 = 16
 // lanes x 32 points only in complex64 (complex128 would hold 64 registers of
 // data per lane and twice the exchange rows)
 template <typename T>
@@ -38,7 +39,9 @@ constexpr int zw_lanes(int N) {
     case 32: return 4;
     case 48: return 4;
     case 64: return 8;
+    case 96: return 4;
     case 128: return 8;
+    case 192: return 8;
     case 256: return 16;
     case 512: return sizeof(T) == 4 ? 16 : 0;
     default: return 0;
@@ -51,8 +54,10 @@ struct ZW {
     static constexpr int B = N / A;
     static constexpr int PW = 64 / A;             // pencils per wave
     static constexpr int ROW = A + 1;             // padded exchange row
-    // exchange rows held at once: all B, or A in two phases when B = 2A > 16
-    static constexpr int XR = (B > 16) ? A : B;
+    // exchange rows held at once: all B, or A in B / A phases where that many points
+    // would take the LDS of a second workgroup per CU
+    static constexpr bool PHASES = B > 16 && (B == 2 * A || sizeof(T) == 8);
+    static constexpr int XR = PHASES ? A : B;
     // exchange elements per pencil: the smallest odd multiple of A that holds
     // the rows, so the 64/A pencils of a wave start at 32/A different
     // 8-byte bank slots and a wave's exchange access is at most 2-way
@@ -100,10 +105,9 @@ __device__ __forceinline__ void zw_fft(cplx<T> (&v)[B], cplx<T>* X, const TwE<T>
     dft<B, S>(v);
 #pragma unroll
     for (int kb = 1; kb < B; kb++) v[kb] = tw_mul<S>(v[kb], tw[kb * A + l]);  // w_N^(l kb)
-    if constexpr (B > 16) {
+    if constexpr (B > 16 && B == 2 * A) {
         // two phases through A rows: columns kb < A, then kb >= A.  The second
         // half is in LDS before the first phase's outputs overwrite its registers.
-        static_assert(B == 2 * A, "two-phase exchange needs B = 2A");
 #pragma unroll
         for (int kb = 0; kb < A; kb++) X[kb * ROW + l] = v[kb];
         wave_lds_sync();
@@ -122,6 +126,24 @@ __device__ __forceinline__ void zw_fft(cplx<T> (&v)[B], cplx<T>* X, const TwE<T>
         dft<A, S>(u);
 #pragma unroll
         for (int ka = 0; ka < A; ka++) v[1 + 2 * ka] = u[ka];
+    } else if constexpr (ZW<T, N>::PHASES) {
+        // B / A phases through A rows; a phase's registers are free once written
+        cplx<T> o[B];
+#pragma unroll
+        for (int m = 0; m < B / A; m++) {
+#pragma unroll
+            for (int kb = 0; kb < A; kb++) X[kb * ROW + l] = v[A * m + kb];
+            wave_lds_sync();
+            cplx<T> u[A];
+#pragma unroll
+            for (int q = 0; q < A; q++) u[q] = X[l * ROW + q];
+            wave_lds_sync();
+            dft<A, S>(u);
+#pragma unroll
+            for (int ka = 0; ka < A; ka++) o[m + (B / A) * ka] = u[ka];
+        }
+#pragma unroll
+        for (int b = 0; b < B; b++) v[b] = o[b];
     } else {
 #pragma unroll
         for (int kb = 0; kb < B; kb++) X[kb * ROW + l] = v[kb];
@@ -634,6 +656,12 @@ unsigned launch_zwave(const PassArgs<T>& a, hipStream_t s) {
         // compiled with the hook file; these kernels carry none of its code
         if (a.axis != 2 || a.nred > 3 || a.ph.modify) return 0;
         const unsigned blocks = (a.M + ZW<T, N>::PENCILS - 1) / ZW<T, N>::PENCILS;
+        // complex128 at 96 and 192 points holds 24 points per lane (256 VGPRs
+        // and some spills), so it pays once the workgroups reach more than half
+        // of the CUs: us per real-time step in LDS tiles / in waves 32x24x96
+        // 36 / 51, 64x64x192 84 / 88 (128 workgroups), 96^3 107 / 98 (144),
+        // 128x128x192 251 / 172, 192^3 551 / 395
+        if (sizeof(T) == 8 && ZW<T, N>::B > 16 && 4 * blocks <= a.pipe_wgs) return 0;
         const int shape = pass_shape(a.dir1, a.dir2);
         const int lm = (a.load_mode == LOAD_PLAIN && (a.flags & F_RED_POT)) ? LOAD_REDPOT : a.load_mode;
         const int mm = a.mid_mode;
