@@ -990,21 +990,10 @@ constexpr bool same_plan(const FftPlan& a, const FftPlan& b) {
 // whether a length has an alternative schedule
 constexpr bool has_alt_plan(int N, bool c64) { return !same_plan(alt_plan(N, c64), make_plan(N, c64)); }
 
-// Radices of four and below: four points per thread, for tiles so few that a
-// workgroup's own chain of instructions is what takes the time (gpe_xcd.hpp)
-constexpr FftPlan fine_plan(int N) {
-    FftPlan p{0, {0, 0, 0, 0, 0, 0, 0, 0}};
-    int n = N;
-    while (n % 4 == 0) { p.r[p.ns++] = 4; n /= 4; }
-    while (n % 3 == 0) { p.r[p.ns++] = 3; n /= 3; }
-    while (n % 2 == 0) { p.r[p.ns++] = 2; n /= 2; }
-    return p;
-}
-
-// plan of a transform: PV 0 the default schedule, 1 the alternative, 2 the fine one; rev
+// plan of a transform: PV 0 the default schedule, 1 the alternative; rev
 // reverses the radix order (the second transform of a turn-around pass)
 constexpr FftPlan plan_of(int N, bool rev, bool c64, int pv = 0) {
-    FftPlan p = pv == 2 ? fine_plan(N) : pv ? alt_plan(N, c64) : make_plan(N, c64);
+    FftPlan p = pv ? alt_plan(N, c64) : make_plan(N, c64);
     if (rev)
         for (int i = 0; i < p.ns / 2; i++) {
             int t = p.r[i];
@@ -1075,38 +1064,6 @@ template <int M, int W, bool CONTIG>
 __device__ __forceinline__ void bmap(int b, int& w, int& j) {
     if constexpr (CONTIG) { w = b / M; j = b % M; }
     else { j = b / W; w = b % W; }
-}
-
-// first stage from global memory (load op applied per element) into LDS
-template <typename T, int N, int W, bool CONTIG, bool FULL, int S, int R, int AX = -1>
-__device__ __forceinline__ void first_stage_global(const PassArgs<T>& a, unsigned p0, cplx<T>* lds, double* acc) {
-    constexpr int M = N / R;
-    constexpr int NB = W * M;
-    constexpr int PER = (NB + kThreads - 1) / kThreads;
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-        const int b = threadIdx.x + q * kThreads;
-        if ((NB % kThreads) == 0 || b < NB) {
-            int w, j;
-            bmap<M, W, CONTIG>(b, w, j);
-            const unsigned p = p0 + (unsigned)w;
-            cplx<T> v[R];
-            if (p < a.M) {
-                const Pencil pc = make_pencil<AX>(a, N, p);
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const Coord c = elem<AX>(a, pc, (unsigned)(j + r * M));
-                    v[r] = a.src[c.off];
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < R; r++) v[r] = mk((T)0, (T)0);
-            }
-            dft<R, S>(v);
-#pragma unroll
-            for (int r = 0; r < R; r++) lds[lidx<T, N, W, CONTIG>(w, j * R + r)] = v[r];
-        }
-    }
 }
 
 // first stage of a lean pass from HBM into the LDS tile, calling pre() once
