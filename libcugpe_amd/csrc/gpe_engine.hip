@@ -183,16 +183,15 @@ void build_kinetic(gpe_engine_s* e) {
 
 // Kinetic factors in FP64; for complex64 also K_x and the products K_y K_z
 // per (iy, iz), each as a float pair hi + lo with hi + lo = K to ~1e-15.
-// conj: the conjugate tables (the adjoint's kinetic step) into the adjoint's
-// own arrays.
-int upload_kinetic_tables(gpe_engine_s* e, bool conj) {
+// conj: the conjugate tables (the adjoint's kinetic step).
+int upload_kinetic_tables(gpe_engine_s* e, bool conj, void* Ktab, void* Khl) {
     auto val = [&](std::complex<double> v) { return conj ? std::conj(v) : v; };
     std::vector<cplx<double>> K;
     for (const auto* t : {&e->Kx, &e->Ky, &e->Kz})
         for (auto& v : *t) K.push_back(mk(val(v).real(), val(v).imag()));
     HIP_TRY(hipStreamSynchronize(e->stream));
-    HIP_TRY(hipMemcpy(conj ? e->adj_Ktab : e->Ktab, K.data(), K.size() * sizeof(cplx<double>), hipMemcpyHostToDevice));
-    if (e->Khl) {
+    HIP_TRY(hipMemcpy(Ktab, K.data(), K.size() * sizeof(cplx<double>), hipMemcpyHostToDevice));
+    if (Khl) {
         std::vector<cplx<float>> h;
         h.reserve(2 * ((size_t)e->nx + (size_t)e->ny * e->nz));
         auto split = [&](std::complex<double> v) {
@@ -203,14 +202,47 @@ int upload_kinetic_tables(gpe_engine_s* e, bool conj) {
         for (auto& v : e->Kx) split(val(v));
         for (int iy = 0; iy < e->ny; iy++)
             for (int iz = 0; iz < e->nz; iz++) split(val(e->Ky[iy] * e->Kz[iz]));
-        HIP_TRY(hipMemcpy(conj ? e->adj_Khl : e->Khl, h.data(), h.size() * sizeof(cplx<float>), hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(Khl, h.data(), h.size() * sizeof(cplx<float>), hipMemcpyHostToDevice));
     }
     return 0;
 }
 
+size_t ktab_bytes(const gpe_engine_s* e) { return (size_t)(e->nx + e->ny + e->nz) * sizeof(cplx<double>); }
+size_t khl_bytes(const gpe_engine_s* e) {
+    return 2 * ((size_t)e->nx + (size_t)e->ny * e->nz) * sizeof(cplx<float>);
+}
+
+void drop_adjoint_tables(gpe_engine_s* e) {
+    if (e->adj_Ktab) (void)hipFree(e->adj_Ktab);
+    if (e->adj_Khl) (void)hipFree(e->adj_Khl);
+    e->adj_Ktab = e->adj_Khl = nullptr;
+}
+
+// The conjugate tables, made by the first adjoint run.  The engine knows them
+// only once both are allocated and filled: after an error the next run makes
+// them again.
+int make_adjoint_tables(gpe_engine_s* e) {
+    if (e->adj_Ktab) return 0;
+    void *k = nullptr, *h = nullptr;
+    int r = (int)hipMalloc(&k, ktab_bytes(e));
+    if (!r && e->Khl) r = (int)hipMalloc(&h, khl_bytes(e));
+    if (!r) r = upload_kinetic_tables(e, true, k, h);
+    if (r) {
+        if (k) (void)hipFree(k);
+        if (h) (void)hipFree(h);
+        return r;
+    }
+    e->adj_Ktab = k;
+    e->adj_Khl = h;
+    return 0;
+}
+
 int upload_kinetic(gpe_engine_s* e) {
-    if (int r = upload_kinetic_tables(e, false)) return r;
-    return e->adj_Ktab ? upload_kinetic_tables(e, true) : 0;
+    if (int r = upload_kinetic_tables(e, false, e->Ktab, e->Khl)) return r;
+    if (!e->adj_Ktab) return 0;
+    const int r = upload_kinetic_tables(e, true, e->adj_Ktab, e->adj_Khl);
+    if (r) drop_adjoint_tables(e);
+    return r;
 }
 
 template <typename T>
@@ -920,10 +952,9 @@ int create_impl(gpe_engine_s** out, const gpe_config_t* cfg, double alpha, doubl
         ALLOC(e->tw[a], (size_t)axis_len(e, a) * 2 * es);
         if (e->precision == GPE_PRECISION_C64) ALLOC(e->twlo[a], (size_t)axis_len(e, a) * 2 * es);
     }
-    ALLOC(e->Ktab, (size_t)(e->nx + e->ny + e->nz) * sizeof(cplx<double>));
+    ALLOC(e->Ktab, ktab_bytes(e));
     ALLOC(e->ktab, (size_t)(e->nx + e->ny + e->nz) * es);
-    if (e->precision == GPE_PRECISION_C64)
-        ALLOC(e->Khl, 2 * ((size_t)e->nx + (size_t)e->ny * e->nz) * sizeof(cplx<float>));
+    if (e->precision == GPE_PRECISION_C64) ALLOC(e->Khl, khl_bytes(e));
     ALLOC(e->vtab, (size_t)(e->nx + e->ny + e->nz) * es);
     ALLOC(e->k64, (size_t)(e->nx + e->ny + e->nz) * sizeof(double));
     // partial sums: the largest grid of any pass times five (three sums of a z pass, one of a y and an x pass)
@@ -1739,11 +1770,7 @@ int adjoint_forward_t(gpe_engine_s* e, int nt, const cuCplx* tgt, int ckpt, doub
         if (!r) r = adj_alloc((void**)p, &have, n, sizeof(double));
     }
     if (r) return r;
-    if (!e->adj_Ktab) {
-        HIP_TRY(hipMalloc(&e->adj_Ktab, (size_t)(e->nx + e->ny + e->nz) * sizeof(cplx<double>)));
-        if (e->Khl) HIP_TRY(hipMalloc(&e->adj_Khl, 2 * ((size_t)e->nx + (size_t)e->ny * e->nz) * sizeof(cplx<float>)));
-        if (int q = upload_kinetic_tables(e, true)) return q;
-    }
+    if ((r = make_adjoint_tables(e))) return r;
     // the predictor ends of a whole segment, or, where they do not fit, of
     // one step (then each is computed again from its step's input)
     if (adj_alloc(&e->adj_phi, &e->adj_phi_len, (size_t)C * n, cs)) {

@@ -1,0 +1,95 @@
+"""Host paths of the adjoint on the host runtime: an allocation or an upload
+that fails leaves nothing half made behind."""
+import pytest
+
+import host_runtime
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    return host_runtime.build(tmp_path_factory.mktemp("host"))
+
+
+FAILING = """
+shape, nt = (8, 8, 12), 4
+psi = np.ones(shape, complex)
+
+def engine():
+    g = E.Engine(shape, 1.0, 0.0, 0.01, 1.0, E.UFG, E.HARMONIC, 0, {prec})
+    g.set_user_params([0.1, 0.1, 0.1])
+    g.set_psi(psi)
+    return g
+
+def forward(g):
+    "uploaded bytes of a forward run, None where it fails"
+    H.hh_reset()
+    try:
+        g.adjoint_forward(nt, psi)
+    except E.GpeError:
+        return None
+    return H.hh_uploaded()
+
+g = engine()
+base = H.hh_blocks()
+first = forward(g)       # with the conjugate tables
+again = forward(g)       # without them
+live = H.hh_blocks() - base
+tables = first - again
+assert tables > 0
+g.close()
+
+failed = 0
+for what in (0, 1):
+    for k in range(1, 40):
+        g = engine()
+        base = H.hh_blocks()
+        H.hh_fail(0 if what else k, k if what else 0)
+        out = forward(g)
+        H.hh_fail(0, 0)
+        if out is None:
+            failed += 1
+            # nothing of the failed run stands in for the tables: the next one uploads what is missing
+            assert forward(g) in (first, again), (what, k)
+            made = H.hh_blocks() - base
+            assert made == live, (what, k, made, live)
+            g.adjoint_backward()
+            H.hh_reset()
+        g.close()
+print("failed", failed)
+assert failed >= 10
+"""
+
+UPLOADS = """
+# after a failed run, the tables of the next one hold the conjugate factors
+import itertools
+shape, nt = (8, 8, 12), 2
+psi = np.ones(shape, complex)
+for what, k in itertools.product((0, 1), range(1, 30)):
+    g = E.Engine(shape, 1.0, 0.0, 0.01, 1.0, E.UFG, E.HARMONIC, 0, {prec})
+    g.set_user_params([0.1, 0.1, 0.1])
+    H.hh_reset()
+    g.set_psi(psi)
+    H.hh_fail(0 if what else k, k if what else 0)
+    total, fails = 0, 0
+    for _ in range(2):
+        H.hh_reset()
+        try:
+            g.adjoint_forward(nt, psi)
+        except E.GpeError:
+            fails += 1
+        H.hh_fail(0, 0)
+        total += H.hh_uploaded()
+    H.hh_reset()
+    g.adjoint_forward(nt, psi)
+    plain = H.hh_uploaded()
+    n = sum(shape) * 16 + (16 * (shape[0] + shape[1] * shape[2]) if {prec} == E.C64 else 0)
+    # the complete tables went up in one of the runs that did not fail
+    assert total >= n + (2 - fails) * plain, (what, k, fails, total, n, plain)
+    g.close()
+"""
+
+
+@pytest.mark.parametrize("prec", ["E.C64", "E.C128"])
+@pytest.mark.parametrize("code", [FAILING, UPLOADS], ids=["allocations", "uploads"])
+def test_failed_forward_run_leaves_no_half_made_tables(runtime, code, prec):
+    host_runtime.run(runtime, code.format(prec=prec))
