@@ -211,9 +211,16 @@ void adj_zwave_kernel(const AdjArgs<T> a) {
                 if constexpr (PASS != ADJ_P2) a.grad[o] = gr[j] + dg;
                 if constexpr (PASS != ADJ_P4) a.vb[o] = vb[j];
             }
-            v[q * CH + j] = from64<T>(u);
+            // P4 ends here: stored at once, or the compiler interleaves the
+            // chunks and spills (412 bytes per lane at 128 points in complex128)
+            if constexpr (PASS == ADJ_P4) {
+                if (ok) a.lam[o] = from64<T>(u);
+            } else {
+                v[q * CH + j] = from64<T>(u);
+            }
         }
     });
+    if constexpr (PASS == ADJ_P4) return;
     if constexpr (PASS != ADJ_P4) zw_fft<T, N, -1, B>(v, X, L.tw, l);
     if (ok) {
 #pragma unroll
@@ -221,11 +228,15 @@ void adj_zwave_kernel(const AdjArgs<T> a) {
     }
 }
 
-// false: the z length has no wave split
+// false: the z length has no wave split, or one of more than 16 points per lane:
+// the parts then leave too few registers and spill, and the pointwise kernels
+// are faster (us a step of a complex64 gradient in waves / pointwise: 8x12x96
+// 195 / 156, 32x64x192 280 / 229, 64x64x512 1089 / 970).  None of these
+// kernels needs scratch memory, which the runtime would allocate at a first
+// launch on a queue, aborting where none is left.
 template <typename T, int N>
 bool launch_adj_zwave(const AdjArgs<T>& a, int pass, hipStream_t s) {
-    // (24 points per lane in complex128 leave no registers for the parts)
-    if constexpr (zw_lanes<T>(N) == 0 || (sizeof(T) == 8 && N > 16 * zw_lanes<T>(N))) {
+    if constexpr (zw_lanes<T>(N) == 0 || N > 16 * zw_lanes<T>(N)) {
         return false;
     } else {
         const dim3 g((a.M + ZW<T, N>::PENCILS - 1) / ZW<T, N>::PENCILS), b(kThreads);

@@ -1683,7 +1683,8 @@ int gpe_engine_energy_dipolar(gpe_engine_t e, int method, double* t, double* edi
 // pointwise parts and the derivation).  The forward run keeps the state every
 // C steps (C = ceil(sqrt(nt)) by default); the backward run recomputes one
 // segment of C states at a time from its checkpoint and walks it backwards:
-// memory C + nt/C states, work one extra forward run.
+// memory 2 C + nt/C states (C + nt/C where the segment's predictor ends are not
+// kept), work one extra forward run.
 
 namespace {
 
@@ -1771,11 +1772,19 @@ int adjoint_forward_t(gpe_engine_s* e, int nt, const cuCplx* tgt, int ckpt, doub
     }
     if (r) return r;
     if ((r = make_adjoint_tables(e))) return r;
-    // the predictor ends of a whole segment, or, where they do not fit, of
-    // one step (then each is computed again from its step's input)
-    if (adj_alloc(&e->adj_phi, &e->adj_phi_len, (size_t)C * n, cs)) {
-        (void)hipGetLastError();
-        if ((r = adj_alloc(&e->adj_phi, &e->adj_phi_len, n, cs))) return r;
+    // The predictor ends of a whole segment where they take at most half of the
+    // memory still free, else of one step (then each is computed again from its
+    // step's input).  They are the run's only optional array: what is left
+    // serves the caller's own arrays beside a gradient and the scratch memory
+    // the runtime takes at kernels' first launches (an allocation that just
+    // fitted left 82 MB, and such a launch aborted the process).
+    if (e->adj_phi_len < (size_t)C * n) {
+        size_t avail = 0, total = 0;
+        const bool room = hipMemGetInfo(&avail, &total) == hipSuccess && (size_t)C * n * cs <= avail / 2;
+        if (!room || adj_alloc(&e->adj_phi, &e->adj_phi_len, (size_t)C * n, cs)) {
+            (void)hipGetLastError();
+            if ((r = adj_alloc(&e->adj_phi, &e->adj_phi_len, n, cs))) return r;
+        }
     }
     // target in the working precision, V_ext as the forward kernels see it
     if ((r = from_host<T>(e, tgt, (cplx<T>*)e->adj_tgt))) return r;

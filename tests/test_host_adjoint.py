@@ -93,3 +93,45 @@ for what, k in itertools.product((0, 1), range(1, 30)):
 @pytest.mark.parametrize("code", [FAILING, UPLOADS], ids=["allocations", "uploads"])
 def test_failed_forward_run_leaves_no_half_made_tables(runtime, code, prec):
     host_runtime.run(runtime, code.format(prec=prec))
+
+
+MEMORY = """
+# room for everything but the predictors, for half of what they ask, and for all of it
+shape, nt = (16, 16, 16), 24
+psi = np.ones(shape, complex)
+state = 16 * 16 ** 3
+
+def gradient(room):
+    "(free memory after the forward run, launches of the backward run) with `room` states free before them"
+    g = E.Engine(shape, 1.0, 0.0, 0.01, 1.0, E.UFG, E.HARMONIC, 0, E.C128)
+    g.set_user_params([0.1, 0.1, 0.1])
+    g.set_psi(psi)
+    H.hh_memory(H.hh_used() + int(room * state) + 8192)  # the kinetic tables too
+    g.adjoint_forward(nt, psi, nt)
+    left = total() - H.hh_used()
+    n = len(launched(g.adjoint_backward))
+    g.close()
+    H.hh_memory(8 << 30)
+    return left / state, n
+
+def total():
+    f, t = ctypes.c_size_t(), ctypes.c_size_t()
+    assert H.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+    return t.value
+
+# one checkpoint, 25 states of the segment, lam, lam0, target, final state, and
+# the FP64 sensitivity, gradient and potential
+arrays = 1 + 25 + 4 + 1.5
+left, kept = gradient(arrays + 3 * nt)
+assert left >= 2 * nt, left
+for room in (1.5, 4, nt, nt + 0.5, 2 * nt - 1):
+    left, n = gradient(arrays + room)
+    assert n > kept, (room, n, kept)      # each predictor computed again
+    assert left >= room - 1, (room, left)  # one state taken
+left, n = gradient(arrays + 2 * nt)
+assert n == kept and left >= nt, (n, kept, left)
+"""
+
+
+def test_kept_predictors_leave_half_of_the_free_memory(runtime):
+    host_runtime.run(runtime, MEMORY)
