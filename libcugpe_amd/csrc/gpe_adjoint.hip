@@ -7,21 +7,26 @@ namespace gpe {
 
 namespace {
 
-// part PASS (ADJ_P2, ADJ_P3, ADJ_P4) on the adjoint state
+// part PASS (ADJ_P2, ADJ_P3, ADJ_P4) on the adjoint state, ADJ_P1 on the states
 template <typename T, int PASS>
-__global__ __launch_bounds__(kThreads) void adj_point_kernel(const AdjArgs<T> a) {
+__global__ __launch_bounds__(kThreads) void adj_point_kernel(const AdjArgs<T> a, size_t n) {
     const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= a.n) return;
-    const cplx<double> p0 = to64(a.psi0[i]), l = to64(a.lam[i]);
+    if (i >= n) return;
+    const cplx<double> p0 = to64(a.psi0[i]);
+    if constexpr (PASS == ADJ_P1) {
+        a.out[i] = from64<T>(adj_part1(a.p, a.vx[i % a.n], p0));
+        return;
+    }
+    const cplx<double> l = to64(a.lam[i]);
     double dg = 0.0;
     if constexpr (PASS == ADJ_P2) {
         double vb;
-        a.lam[i] = from64<T>(adj_part2(a.p, a.vx[i], p0, to64(a.psi1[i]), to64(a.phi3[i]), l, vb));
+        a.lam[i] = from64<T>(adj_part2(a.p, a.vx[i], p0, to64(a.psi1[i]), to64(a.phi[i]), l, vb));
         a.vb[i] = vb;
     } else if constexpr (PASS == ADJ_P3) {
         double vb = a.vb[i];
         cplx<double> l0;
-        a.lam[i] = from64<T>(adj_part3(a.p, a.vx[i], p0, to64(a.phi3[i]), l, vb, l0, dg));
+        a.lam[i] = from64<T>(adj_part3(a.p, a.vx[i], p0, to64(a.phi[i]), l, vb, l0, dg));
         a.lam0[i] = from64<T>(l0);
         a.vb[i] = vb;
         a.grad[i] += dg;
@@ -76,11 +81,13 @@ inline dim3 grid_of(size_t n) { return dim3((unsigned)((n + kThreads - 1) / kThr
 }  // namespace
 
 template <typename T>
-void launch_adjoint_point(const AdjArgs<T>& a, int part, hipStream_t s) {
+void launch_adjoint_point(const AdjArgs<T>& a, int part, size_t n, hipStream_t s) {
+    const dim3 g = grid_of(n), b(kThreads);
     switch (part) {
-    case ADJ_P2: hipLaunchKernelGGL((adj_point_kernel<T, ADJ_P2>), grid_of(a.n), dim3(kThreads), 0, s, a); break;
-    case ADJ_P3: hipLaunchKernelGGL((adj_point_kernel<T, ADJ_P3>), grid_of(a.n), dim3(kThreads), 0, s, a); break;
-    default: hipLaunchKernelGGL((adj_point_kernel<T, ADJ_P4>), grid_of(a.n), dim3(kThreads), 0, s, a); break;
+    case ADJ_P1: hipLaunchKernelGGL((adj_point_kernel<T, ADJ_P1>), g, b, 0, s, a, n); break;
+    case ADJ_P2: hipLaunchKernelGGL((adj_point_kernel<T, ADJ_P2>), g, b, 0, s, a, n); break;
+    case ADJ_P3: hipLaunchKernelGGL((adj_point_kernel<T, ADJ_P3>), g, b, 0, s, a, n); break;
+    default: hipLaunchKernelGGL((adj_point_kernel<T, ADJ_P4>), g, b, 0, s, a, n); break;
     }
 }
 
@@ -106,7 +113,7 @@ void launch_adjoint_lam_init(void* lam, const void* tgt, double fr, double fi, s
 }
 
 #define GPE_ADJ_INST(T)                                                                                      \
-    template void launch_adjoint_point<T>(const AdjArgs<T>&, int, hipStream_t);                               \
+    template void launch_adjoint_point<T>(const AdjArgs<T>&, int, size_t, hipStream_t);                       \
     template void launch_adjoint_vfill<T>(const Phys<T>&, double*, size_t, hipStream_t);                     \
     template int launch_adjoint_overlap<T>(const void*, const void*, const void*, size_t, double*, hipStream_t); \
     template void launch_adjoint_lam_init<T>(void*, const void*, double, double, size_t, hipStream_t);

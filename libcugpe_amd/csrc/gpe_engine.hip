@@ -90,7 +90,7 @@ struct gpe_engine_s {
     void *adj_ck = nullptr, *adj_seg = nullptr;  // checkpoints, one segment of states
     size_t adj_ck_len = 0, adj_seg_len = 0;     // in states
     void *adj_lam = nullptr, *adj_lam0 = nullptr, *adj_tgt = nullptr, *adj_fin = nullptr;
-    void* adj_phi = nullptr;      // predictor ends of a segment's steps, or of one step (adj_phi_len in states)
+    void* adj_phi = nullptr;      // predictors of a segment's steps, or of one step (adj_phi_len in points)
     size_t adj_phi_len = 0;
     void *adj_Ktab = nullptr, *adj_Khl = nullptr;  // conjugate kinetic factors
     double *adj_vb = nullptr, *adj_grad = nullptr, *adj_vx = nullptr;
@@ -363,6 +363,7 @@ struct PassSpec {
     void* dst;
     int dir1, dir2;
     int load, mid, store, flags, nred;
+    size_t lattices = 0;  // stored one after another; 0: the engine's
 };
 
 // launches one pass; returns the workgroup count (for the reduction finalize)
@@ -370,7 +371,7 @@ template <typename T>
 int run_pass(gpe_engine_s* e, PassArgs<T> a, const PassSpec& s) {
     a.axis = s.axis;
     const int N = axis_len(e, s.axis);
-    a.M = (unsigned)(e->n * e->batch / (size_t)N);
+    a.M = (unsigned)(e->n * (s.lattices ? s.lattices : e->batch) / (size_t)N);
     a.variant = e->variant;
     a.pipe_wgs = 2u * (unsigned)e->cus;
     a.n1 = (unsigned)e->n;
@@ -425,13 +426,12 @@ int normalize_t(gpe_engine_s* e) {
 // step but the last ends in a pass that also opens the next one.
 // pin: 0 none, 1 vortex imprint, 2 imprint where |psi| > 1e-15, 3 stored phase;
 // mid_pin: re-applied after the predictor normalisation in imaginary time
-// psi0, psi1, phi3 (real time without pinning or friction): where the step reads its state,
-// leaves it, and stores its predictor end; null: in psi, in psi, not at all.
-// psi is then the corrector's work array.
+// psi0, psi1 (real time without pinning or friction): where the step reads its
+// state and leaves it; null: in psi.  psi is then the corrector's work array.
 struct StepPlan {
     int pin = 0;
     bool mid_pin = false;
-    void *psi0 = nullptr, *psi1 = nullptr, *phi3 = nullptr;
+    void *psi0 = nullptr, *psi1 = nullptr;
 };
 
 template <typename T>
@@ -444,7 +444,6 @@ PassArgs<T> step_args(gpe_engine_s* e, const StepPlan& sp) {
     // captured step graph stays valid for every step it is replayed for
     if (e->uses_hooks) a.ph.itp = e->itdev;
     if (sp.psi0) a.psiA = (cplx<T>*)sp.psi0;
-    a.phi3 = (cplx<T>*)sp.phi3;
     return a;
 }
 
@@ -504,15 +503,15 @@ void issue_open(gpe_engine_s* e, const StepPlan& sp) {
 // and x (forward x, K_x, inverse x).  Launcher variant bit 3 selects the
 // unsplit plan: forward y, the x turn-around with K_x K_y K_z, inverse y.
 template <typename T>
-void kinetic_kz(gpe_engine_s* e, const PassArgs<T>& a, void* buf) {
+void kinetic_kz(gpe_engine_s* e, const PassArgs<T>& a, void* buf, size_t lattices = 0) {
     const int F = -1, I = +1;
     if (!(e->variant & 8)) {
-        run_pass<T>(e, a, {1, buf, buf, F, I, LOAD_PLAIN, MID_EXPT_SEP, STORE_PLAIN, 0, 0});
-        run_pass<T>(e, a, {0, buf, buf, F, I, LOAD_PLAIN, MID_EXPT_SEP, STORE_PLAIN, 0, 0});
+        run_pass<T>(e, a, {1, buf, buf, F, I, LOAD_PLAIN, MID_EXPT_SEP, STORE_PLAIN, 0, 0, lattices});
+        run_pass<T>(e, a, {0, buf, buf, F, I, LOAD_PLAIN, MID_EXPT_SEP, STORE_PLAIN, 0, 0, lattices});
     } else {
-        run_pass<T>(e, a, {1, buf, buf, F, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
-        run_pass<T>(e, a, {0, buf, buf, F, I, LOAD_PLAIN, MID_EXPT, STORE_PLAIN, 0, 0});
-        run_pass<T>(e, a, {1, buf, buf, I, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
+        run_pass<T>(e, a, {1, buf, buf, F, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0, lattices});
+        run_pass<T>(e, a, {0, buf, buf, F, I, LOAD_PLAIN, MID_EXPT, STORE_PLAIN, 0, 0, lattices});
+        run_pass<T>(e, a, {1, buf, buf, I, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0, lattices});
     }
 }
 
@@ -524,7 +523,7 @@ void issue_step(gpe_engine_s* e, const StepPlan& sp, bool last) {
         const PassArgs<T> a = step_args<T>(e, sp);
         void *A = e->A, *B = e->B;
         run_pass<T>(e, a, {0, B, B, -1, +1, LOAD_PLAIN, MID_EXPT_SEP, STORE_PLAIN, 0, 0});
-        plane_run<T>(e, a, sp.phi3 ? PL_VSTEP2P : PL_VSTEP2, B, A, 0);
+        plane_run<T>(e, a, PL_VSTEP2, B, A, 0);
         run_pass<T>(e, a, {0, A, A, -1, +1, LOAD_PLAIN, MID_EXPT_SEP, STORE_PLAIN, 0, 0});
         const PassArgs<T> a1 = end_args<T>(e, a, sp);
         if (!last) plane_run<T>(e, a1, PL_VSTEP3_NEXT, A, B, F_NEXT_VSTEP1);
@@ -549,7 +548,7 @@ void issue_step(gpe_engine_s* e, const StepPlan& sp, bool last) {
     // predictor kinetic step of phi1
     kinetic_kz<T>(e, a, B);
     if (!ite) {
-        run_pass<T>(e, a, {2, B, A, I, F, LOAD_PLAIN, sp.phi3 ? MID_VSTEP2P : MID_VSTEP2, STORE_PLAIN, fqf, 0});
+        run_pass<T>(e, a, {2, B, A, I, F, LOAD_PLAIN, MID_VSTEP2, STORE_PLAIN, fqf, 0});
     } else {
         const int nb = run_pass<T>(e, a, {2, B, B, I, 0, LOAD_PLAIN, MID_PART1, STORE_PLAIN, fqf, 1});
         finalize(e, nb, 1, FIN_NORM, 0, 1.0);
@@ -1683,7 +1682,7 @@ int gpe_engine_energy_dipolar(gpe_engine_t e, int method, double* t, double* edi
 // pointwise parts and the derivation).  The forward run keeps the state every
 // C steps (C = ceil(sqrt(nt)) by default); the backward run recomputes one
 // segment of C states at a time from its checkpoint and walks it backwards:
-// memory 2 C + nt/C states (C + nt/C where the segment's predictor ends are not
+// memory 2 C + nt/C states (C + nt/C where the segment's predictors are not
 // kept), work one extra forward run.
 
 namespace {
@@ -1698,16 +1697,14 @@ int adj_alloc(void** p, size_t* have, size_t want, size_t unit) {
     return 0;
 }
 
-// nt real-time steps from the state at `from`: step j leaves its state at
-// to(j) and its predictor end at phi(j) (null: not stored)
-template <typename T, typename To, typename Phi>
-void adj_steps(gpe_engine_s* e, int nt, void* from, To&& to, Phi&& phi) {
+// nt real-time steps from the state at `from`: step j leaves its state at to(j)
+template <typename T, typename To>
+void adj_steps(gpe_engine_s* e, int nt, void* from, To&& to) {
     StepPlan sp;
     sp.psi0 = from;
     issue_open<T>(e, sp);
     for (int j = 0; j < nt; j++) {
         sp.psi1 = to(j);
-        sp.phi3 = phi(j);
         issue_step<T>(e, sp, j == nt - 1);
         sp.psi0 = sp.psi1;
     }
@@ -1730,7 +1727,7 @@ AdjArgs<T> adj_args(gpe_engine_s* e) {
     a.grad = e->adj_grad;
     a.tw = (const cplx<T>*)e->tw[2];
     a.twlo = (const cplx<T>*)e->twlo[2];
-    a.M = (unsigned)(e->n / (size_t)e->nz);
+    a.M = a.M1 = (unsigned)(e->n / (size_t)e->nz);
     return a;
 }
 
@@ -1742,15 +1739,36 @@ void adj_zpass(gpe_engine_s* e, const AdjArgs<T>& a, int pass) {
     if (!(e->variant & 1) && launch_adjoint_z<T>(e->nz, a, pass, e->stream)) return;
     const PassArgs<T> b = base_args<T>(e);
     if (pass != ADJ_P2) run_pass<T>(e, b, {2, a.lam, a.lam, 1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
-    launch_adjoint_point<T>(a, pass == ADJ_P4P2 ? ADJ_P4 : pass, e->stream);
+    launch_adjoint_point<T>(a, pass == ADJ_P4P2 ? ADJ_P4 : pass, e->n, e->stream);
     if (pass == ADJ_P4P2) {
         AdjArgs<T> c = a;
         c.psi1 = a.psi0;
         c.psi0 = a.psi0p;
-        c.phi3 = a.phi3p;
-        launch_adjoint_point<T>(c, ADJ_P2, e->stream);
+        c.phi = a.phip;
+        launch_adjoint_point<T>(c, ADJ_P2, e->n, e->stream);
     }
     if (pass != ADJ_P4) run_pass<T>(e, b, {2, a.lam, a.lam, -1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0});
+}
+
+// The predictors phi of `count` steps from their states at psi0, into phi (both
+// stored one after another): P1 and a kinetic step
+template <typename T>
+void adj_predictors(gpe_engine_s* e, const PassArgs<T>& fwd, const cplx<T>* psi0, cplx<T>* phi, size_t count) {
+    // offsets within a pass are 32-bit
+    const size_t most = std::max((size_t)1, (((size_t)1 << 31) - 1) / e->n);
+    for (size_t done = 0; done < count; done += most) {
+        const size_t k = std::min(most, count - done);
+        AdjArgs<T> a = adj_args<T>(e);
+        a.psi0 = psi0 + done * e->n;
+        a.out = phi + done * e->n;
+        a.M = a.M1 * (unsigned)k;
+        if ((e->variant & 1) || !launch_adjoint_z<T>(e->nz, a, ADJ_P1, e->stream)) {
+            launch_adjoint_point<T>(a, ADJ_P1, k * e->n, e->stream);
+            run_pass<T>(e, fwd, {2, a.out, a.out, -1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0, k});
+        }
+        kinetic_kz<T>(e, fwd, a.out, k);
+        run_pass<T>(e, fwd, {2, a.out, a.out, 1, 0, LOAD_PLAIN, MID_NONE, STORE_PLAIN, 0, 0, k});
+    }
 }
 
 template <typename T>
@@ -1772,9 +1790,8 @@ int adjoint_forward_t(gpe_engine_s* e, int nt, const cuCplx* tgt, int ckpt, doub
     }
     if (r) return r;
     if ((r = make_adjoint_tables(e))) return r;
-    // The predictor ends of a whole segment where they take at most half of the
-    // memory still free, else of one step (then each is computed again from its
-    // step's input).  They are the run's only optional array: what is left
+    // The predictors of a whole segment where they take at most half of the
+    // memory still free, else of one step.  They are the run's only optional array: what is left
     // serves the caller's own arrays beside a gradient and the scratch memory
     // the runtime takes at kernels' first launches (an allocation that just
     // fitted left 82 MB, and such a launch aborted the process).
@@ -1795,8 +1812,7 @@ int adjoint_forward_t(gpe_engine_s* e, int nt, const cuCplx* tgt, int ckpt, doub
         [&](int j) -> void* {
             const int k = j + 1;  // the state's time index
             return (k % C == 0 && k < nt) ? (char*)e->adj_ck + (size_t)(k / C) * n * cs : (char*)e->A;
-        },
-        [](int) -> void* { return nullptr; });
+        });
     e->it += (unsigned)nt;
     const int nb = launch_adjoint_overlap<T>(e->A, e->adj_tgt, e->adj_ck, n, e->partials, e->stream);
     HIP_TRY(hipGetLastError());
@@ -1842,20 +1858,14 @@ int adjoint_backward_t(gpe_engine_s* e, double* grad, bool device_out = false) {
     for (int sg = nck - 1; sg >= 0; sg--) {
         const int k0 = sg * C, len = std::min(nt, k0 + C) - k0;
         HIP_TRY(hipMemcpyAsync(seg, (cplx<T>*)e->adj_ck + (size_t)sg * n, n * cs, hipMemcpyDeviceToDevice, e->stream));
-        adj_steps<T>(
-            e, len, seg, [&](int j) -> void* { return seg + (size_t)(j + 1) * n; },
-            [&](int j) -> void* { return stored ? phi + (size_t)j * n : nullptr; });
-        // the predictor end of step j of the segment
+        adj_steps<T>(e, len, seg, [&](int j) -> void* { return seg + (size_t)(j + 1) * n; });
+        if (stored) adj_predictors<T>(e, fwd, seg, phi, (size_t)len);
         auto predictor = [&](int j) -> const cplx<T>* {
             if (stored) return phi + (size_t)j * n;
-            PassArgs<T> f = fwd;
-            f.psiA = seg + (size_t)j * n;
-            run_pass<T>(e, f, {2, nullptr, e->B, -1, 0, LOAD_PSI0, MID_NONE, STORE_PLAIN, F_VSTEP1, 0});
-            kinetic_kz<T>(e, f, e->B);
-            run_pass<T>(e, f, {2, e->B, phi, 1, 0, LOAD_PLAIN, MID_PART1, STORE_PLAIN, 0, 0});
+            adj_predictors<T>(e, fwd, seg + (size_t)j * n, phi, 1);
             return phi;
         };
-        a.phi3 = predictor(len - 1);
+        a.phi = predictor(len - 1);
         for (int j = len - 1; j >= 0; j--) {
             a.psi0 = seg + (size_t)j * n;
             a.psi1 = seg + (size_t)(j + 1) * n;
@@ -1865,9 +1875,9 @@ int adjoint_backward_t(gpe_engine_s* e, double* grad, bool device_out = false) {
             kinetic_kz<T>(e, rev, a.lam);
             if (j > 0) {
                 a.psi0p = seg + (size_t)(j - 1) * n;
-                a.phi3p = predictor(j - 1);
+                a.phip = predictor(j - 1);
                 adj_zpass<T>(e, a, ADJ_P4P2);
-                a.phi3 = a.phi3p;
+                a.phi = a.phip;
             } else {
                 adj_zpass<T>(e, a, ADJ_P4);
             }

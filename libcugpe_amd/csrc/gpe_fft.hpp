@@ -446,7 +446,6 @@ enum MidMode {
     MID_DIP_STEP = 14,   // psi exp(c (Vext + Vdip)), Vdip the real part of the value (dev/gpe_engine.cu:984-1008)
     MID_DIP_RHO = 15,    // psi stored, its density goes on (dev/gpe_engine.cu:618-626)
     MID_DIP_E2 = 16,     // sum rho Vdip (dev/gpe_engine.cu:1768-1782)
-    MID_VSTEP2P = 17,    // MID_VSTEP2 that also stores phi3 (the adjoint's recomputed steps)
 };
 
 // Fourier transform of the particle-particle potential of z-polarised dipoles
@@ -490,7 +489,6 @@ struct PassArgs {
     const cplx<T>* twlo;   // complex64: exp(-2 pi i m / N) - tw, the low part
     cplx<T>* psiA;         // the wave function buffer (psi0 / psi1)
     T* vbuf;               // corrector potential V1 per point
-    cplx<T>* phi3;         // predictor end per point (MID_VSTEP2P)
     T* vq;                 // quantum-friction potential per point
     double* rout;          // real FP64 output (currents)
     const cplx<double>* Kx;  // kinetic factors in FP64, Kz includes 1/N
@@ -829,12 +827,11 @@ template <int MM, bool UH = false, typename T>
 __device__ __forceinline__ cplx<T> mid_op_m(const PassArgs<T>& a, const ElemIn<T>& e, cplx<T> v, double* acc) {
     const bool qf = (a.flags & F_QF) != 0;
     const unsigned off = e.c.off;
-    if constexpr (MM == MID_VSTEP2 || MM == MID_VSTEP2P) {
+    if constexpr (MM == MID_VSTEP2) {
         // orginal/gpe_engine.cu:774-801 (and the _part1/_part2[_qf] pair for qf)
         const cplx<T> psi0 = modify_at<UH>(a, e, e.aux, e.it);
         const T V0 = pot2<UH>(a, e.vx, psi0, qf, e.raux, e.it, off);
         const cplx<T> phi3 = mul_exp(v, a.ph.c.x * V0, a.ph.c.y * V0);
-        if constexpr (MM == MID_VSTEP2P) a.phi3[off] = phi3;
         T lv;
         const T d1 = dedfdn<UH>(a.ph, density(a.ph, phi3), e.it + 1, off);
         if (qf) lv = (T)0.5 * (V0 + e.vx1 + d1 + e.raux);
@@ -910,7 +907,6 @@ template <bool UH, typename T>
 __device__ __forceinline__ cplx<T> mid_op2(const PassArgs<T>& a, const ElemIn<T>& e, cplx<T> v, double* acc) {
     switch (a.mid_mode) {
     case MID_VSTEP2: return mid_op_m<MID_VSTEP2, UH>(a, e, v, acc);
-    case MID_VSTEP2P: return mid_op_m<MID_VSTEP2P, UH>(a, e, v, acc);
     case MID_PART1: return mid_op_m<MID_PART1, UH>(a, e, v, acc);
     case MID_VSTEP3: return mid_op_m<MID_VSTEP3, UH>(a, e, v, acc);
     case MID_QF_VSTEP1: return mid_op_m<MID_QF_VSTEP1, UH>(a, e, v, acc);
@@ -1465,7 +1461,7 @@ template <typename T>
 __device__ __forceinline__ bool needs_psi0(const PassArgs<T>& a) {
     return a.load_mode == LOAD_PART2 || a.mid_mode == MID_VSTEP2 || a.mid_mode == MID_PART1 ||
            a.mid_mode == MID_QF_VSTEP1 || a.mid_mode == MID_OVERLAP_RE || a.mid_mode == MID_DIP_STEP ||
-           a.mid_mode == MID_DIP_E2 || a.mid_mode == MID_VSTEP2P;
+           a.mid_mode == MID_DIP_E2;
 }
 template <typename T>
 __device__ __forceinline__ const T* real_side(const PassArgs<T>& a) {

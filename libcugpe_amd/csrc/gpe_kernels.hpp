@@ -145,10 +145,10 @@ bool plane_length_ok(int L);
 template <typename T>
 int launch_plane(const PassArgs<T>& a, int L, int mode, unsigned planes, bool uh, hipStream_t s);
 
-// discrete adjoint of the real-time split step: part P2, P3 or P4 of a
-// backward step as a pointwise kernel (gpe_adjoint.hip)
+// discrete adjoint of the real-time split step: part P1, P2, P3 or P4 of a
+// backward step as a pointwise kernel over n points (gpe_adjoint.hip)
 template <typename T>
-void launch_adjoint_point(const AdjArgs<T>& a, int part, hipStream_t s);
+void launch_adjoint_point(const AdjArgs<T>& a, int part, size_t n, hipStream_t s);
 template <typename T>
 void launch_adjoint_vfill(const Phys<T>& ph, double* out, size_t n, hipStream_t s);
 // partials [4][nb]: Re, Im of sum conj(tgt) psi, sum |a0|^2, sum |tgt|^2; nb returned

@@ -10,10 +10,6 @@ void launch_mode(const PassArgs<T>& a, int mode, unsigned planes, hipStream_t s)
     const dim3 g(planes), b(plane_threads<L>());
     switch (mode) {
     case PL_OPEN: hipLaunchKernelGGL((plane_kernel<T, L, PL_OPEN, UH>), g, b, 0, s, a); break;
-    // the adjoint's recomputed steps (no user hooks)
-    case PL_VSTEP2P:
-        if constexpr (!UH) hipLaunchKernelGGL((plane_kernel<T, L, PL_VSTEP2P, false>), g, b, 0, s, a);
-        break;
     case PL_VSTEP2: hipLaunchKernelGGL((plane_kernel<T, L, PL_VSTEP2, UH>), g, b, 0, s, a); break;
     case PL_VSTEP3_NEXT: hipLaunchKernelGGL((plane_kernel<T, L, PL_VSTEP3_NEXT, UH>), g, b, 0, s, a); break;
     default: hipLaunchKernelGGL((plane_kernel<T, L, PL_VSTEP3_LAST, UH>), g, b, 0, s, a); break;

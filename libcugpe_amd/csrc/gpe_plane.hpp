@@ -52,8 +52,7 @@ __device__ __forceinline__ void pot_chunk(const Phys<T>& p, const cplx<T> (&v)[C
     }
 }
 
-// PL_VSTEP2P: PL_VSTEP2 that also stores the predictor end phi3
-enum PlaneMode { PL_OPEN = 0, PL_VSTEP2 = 1, PL_VSTEP3_NEXT = 2, PL_VSTEP3_LAST = 3, PL_VSTEP2P = 4 };
+enum PlaneMode { PL_OPEN = 0, PL_VSTEP2 = 1, PL_VSTEP3_NEXT = 2, PL_VSTEP3_LAST = 3 };
 
 // threads of a plane workgroup: 512 for 64 x 64 planes (one butterfly of the
 // last stage per thread), 256 otherwise
@@ -267,7 +266,6 @@ __device__ __forceinline__ void plane_tile(const PassArgs<T>& a, PlaneLds<T, L>&
         if constexpr (L2) *p = w;
         else st_nt(p, w);
     };
-    constexpr bool V2 = (MODE == PL_VSTEP2 || MODE == PL_VSTEP2P);
 
     if constexpr (MODE == PL_OPEN) {
         // psi0 with the step's Vstep1 (orginal/gpe_engine.cu:723-772), row-major
@@ -302,8 +300,8 @@ __device__ __forceinline__ void plane_tile(const PassArgs<T>& a, PlaneLds<T, L>&
         __syncthreads();
     } else {
         // side inputs of the physics at this thread's last-stage elements, loaded early
-        cplx<T> side_c[V2 ? PER : 1][V2 ? R : 1];
-        T side_r[V2 ? 1 : PER][V2 ? 1 : R];
+        cplx<T> side_c[MODE == PL_VSTEP2 ? PER : 1][MODE == PL_VSTEP2 ? R : 1];
+        T side_r[MODE == PL_VSTEP2 ? 1 : PER][MODE == PL_VSTEP2 ? 1 : R];
 #pragma unroll
         for (int q = 0; q < PER; q++) {
             const int b = tid + q * kPlaneThreads;
@@ -312,7 +310,7 @@ __device__ __forceinline__ void plane_tile(const PassArgs<T>& a, PlaneLds<T, L>&
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     const unsigned off = base + (unsigned)((j + r * M) * L + w);
-                    if constexpr (V2) side_c[q][r] = side_ld(a.psiA + off);
+                    if constexpr (MODE == PL_VSTEP2) side_c[q][r] = side_ld(a.psiA + off);
                     else side_r[q][r] = side_ld(a.vbuf + off);
                 }
             }
@@ -333,7 +331,7 @@ __device__ __forceinline__ void plane_tile(const PassArgs<T>& a, PlaneLds<T, L>&
             const int w = b % L, j = b / L;
             T vx[R], gv[R], lv[R];
             if constexpr (!UH) plane_vext<false, T, R, M>(a, ix, w, j, base, it, sep, vscale, vx);
-            if constexpr (V2) {
+            if constexpr (MODE == PL_VSTEP2) {
                 // predictor end and corrector potential (orginal/gpe_engine.cu:774-801)
                 if constexpr (!UH) {
                     cplx<T> p0[R];
@@ -344,10 +342,6 @@ __device__ __forceinline__ void plane_tile(const PassArgs<T>& a, PlaneLds<T, L>&
 #pragma unroll
                     for (int r = 0; r < R; r++) gv[r] = V0[r] + vx[r];
                     mul_exp_chunk(v[q], V0, cx, cy);  // phi3
-                    if constexpr (MODE == PL_VSTEP2P) {
-#pragma unroll
-                        for (int r = 0; r < R; r++) side_st(a.phi3 + base + (unsigned)((j + r * M) * L + w), v[q][r]);
-                    }
                     pot_chunk(a.ph, v[q], gv, lv);
 #pragma unroll
                     for (int r = 0; r < R; r++) {

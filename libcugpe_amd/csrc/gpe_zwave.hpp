@@ -365,13 +365,13 @@ __device__ __forceinline__ void zwave_tile(const PassArgs<T>& a, const TwE<T>* t
     static_assert(NCH * CH == B, "chunks must tile the points of a lane");
     constexpr bool PRE = (LM != LOAD_PLAIN);   // physics before the first transform
     constexpr bool POST = (MM != MID_NONE && MM != MID_KAX_SUM);  // physics after it
-    constexpr bool NEED_AUX = (LM == LOAD_PART2) || MM == MID_VSTEP2 || MM == MID_VSTEP2P || MM == MID_PART1 ||
+    constexpr bool NEED_AUX = (LM == LOAD_PART2) || MM == MID_VSTEP2 || MM == MID_PART1 ||
                               MM == MID_QF_VSTEP1 || MM == MID_OVERLAP_RE || MM == MID_DIP_STEP ||
                               MM == MID_DIP_E2;
     const T* rs = real_side(a);
     const bool qf = (a.flags & F_QF) != 0;
     // the fast chunk forms: ops without imprint, built-in physics
-    const bool fast = (MM == MID_VSTEP2) || (MM == MID_VSTEP2P) || (MM == MID_VSTEP3 && !(a.flags & F_IMPRINT_NEXT)) ||
+    const bool fast = (MM == MID_VSTEP2) || (MM == MID_VSTEP3 && !(a.flags & F_IMPRINT_NEXT)) ||
                       (LM == LOAD_PSI0 && !(a.flags & F_IMPRINT)) || (LM == LOAD_PART2 && !(a.flags & F_IMPRINT_MID)) ||
                       MM == MID_PART1 || MM == MID_QF_VSTEP1 || LM == LOAD_RHO || MM == MID_DIP_STEP ||
                       MM == MID_DIP_RHO || MM == MID_DIP_E2;
@@ -469,7 +469,7 @@ __device__ __forceinline__ void zwave_tile(const PassArgs<T>& a, const TwE<T>* t
                     for (int j = 0; j < CH; j++)
                         acc[0] += dens64((double)a.ph.gamma, (double)ax[slot][j].x, (double)ax[slot][j].y) * (double)u[j].x;
                 }
-            } else if constexpr (MM == MID_VSTEP2 || MM == MID_VSTEP2P) {
+            } else if constexpr (MM == MID_VSTEP2) {
                 // predictor end and corrector potential (orginal/gpe_engine.cu:774-801)
                 cplx<T> p0[CH];
 #pragma unroll
@@ -479,12 +479,6 @@ __device__ __forceinline__ void zwave_tile(const PassArgs<T>& a, const TwE<T>* t
 #pragma unroll
                 for (int j = 0; j < CH; j++) V0[j] = vx[j] + gv[j] + (qf ? rx[slot][j] : (T)0);
                 mul_exp_chunk(u, V0, a.ph.c.x, a.ph.c.y);  // phi3
-                if constexpr (MM == MID_VSTEP2P) {
-                    if (ok) {
-#pragma unroll
-                        for (int j = 0; j < CH; j++) st(&a.phi3[off_of(q * CH + j)], u[j]);
-                    }
-                }
                 dedfdn_chunk(a.ph, u, gv);
 #pragma unroll
                 for (int j = 0; j < CH; j++) lv[j] = (T)0.5 * (V0[j] + vx[j] + gv[j] + (qf ? rx[slot][j] : (T)0));
@@ -679,7 +673,6 @@ unsigned launch_zwave(const PassArgs<T>& a, hipStream_t s) {
         GPE_ZW(SHAPE_I, LOAD_PLAIN, MID_VSTEP3)
         GPE_ZW(SHAPE_I, LOAD_PLAIN, MID_OVERLAP_RE)
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_VSTEP2)
-        GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_VSTEP2P)
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_VSTEP3)
         GPE_ZW(SHAPE_IF, LOAD_PLAIN, MID_QF_VSTEP1)
         GPE_ZW(SHAPE_F, LOAD_RHO, MID_NONE)
