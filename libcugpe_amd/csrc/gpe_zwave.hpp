@@ -25,8 +25,8 @@
 
 namespace gpe {
 
-// lanes per pencil; 0: the length runs in the LDS-tile kernels (96 and 192 points in
-// complex64 against those, us per step: 96^3 72 -> 69, 128x128x192 129 -> 96, 192^3 268 -> 218).  512 = 16
+// lanes per pencil; 0: the length runs in the LDS-tile kernels (96 and 192 points
+// run in either, zw_takes).  512 = 16
 // lanes x 32 points only in complex64 (complex128 would hold 64 registers of
 // data per lane and twice the exchange rows)
 template <typename T>
@@ -370,9 +370,12 @@ __device__ __forceinline__ void zwave_tile(const PassArgs<T>& a, const TwE<T>* t
                               MM == MID_DIP_E2;
     const T* rs = real_side(a);
     const bool qf = (a.flags & F_QF) != 0;
-    // the fast chunk forms: ops without imprint, built-in physics
-    const bool fast = (MM == MID_VSTEP2) || (MM == MID_VSTEP3 && !(a.flags & F_IMPRINT_NEXT)) ||
-                      (LM == LOAD_PSI0 && !(a.flags & F_IMPRINT)) || (LM == LOAD_PART2 && !(a.flags & F_IMPRINT_MID)) ||
+    // the fast chunk forms: ops without imprint (which never comes here in
+    // complex64 at 24 points per lane, zw_takes), built-in physics
+    constexpr bool PINS = B != 24 || sizeof(T) == 8;
+    const bool fast = (MM == MID_VSTEP2) || (MM == MID_VSTEP3 && !(PINS && (a.flags & F_IMPRINT_NEXT))) ||
+                      (LM == LOAD_PSI0 && !(PINS && (a.flags & F_IMPRINT))) ||
+                      (LM == LOAD_PART2 && !(PINS && (a.flags & F_IMPRINT_MID))) ||
                       MM == MID_PART1 || MM == MID_QF_VSTEP1 || LM == LOAD_RHO || MM == MID_DIP_STEP ||
                       MM == MID_DIP_RHO || MM == MID_DIP_E2;
     cplx<T> ax[2][CH];
@@ -638,6 +641,44 @@ void zwave_kernel(const PassArgs<T> a) {
     }
 }
 
+// Whether a z pass of a length with a wave split takes it.  Always but at 24
+// points per lane; there (96 and 192 points) a lane's state leaves two workgroups
+// per CU and spills in complex128, so it depends on the pass.  us per step in
+// waves / LDS tiles of the whole step, `blocks` the workgroups of waves on 256
+// CUs (two per CU: 512):
+//   plain and contact passes: complex64 always (8x12x96 37 / 41, 128x128x192
+//     96 / 127, imaginary time 55 / 62), complex128 above 128 blocks (144: real
+//     time 101 / 111, imaginary 139 / 159; 64x64x192, 128: 88 / 84)
+//   unitary gas (pow23 two to four times a point): complex64 above 256 blocks
+//     (128x128x96, 256: 102 / 86, imaginary 141 / 119, friction 147 / 131;
+//     288: 115 / 118, 160 / 163, 169 / 178; 1152: 267 / 276), complex128 above
+//     170 (144: 122 / 114; 192: 135 / 134, imaginary 176 / 182)
+//   extended Thomas-Fermi (two pows) and pinned passes (atan2, hypot, sincos;
+//     not in the chunked form): where the last round of workgroups is more than
+//     three quarters full (ETF complex128 512: 260 / 319, 288: 223 / 199, 576:
+//     413 / 374, 144: 195 / 131; complex64 512: 151 / 163, 1152: 389 / 340, 256:
+//     140 / 106), the pinned ones only in complex128 (all passes of a step with
+//     a vortex line, complex128 512: 318 / 419, 144: 236 / 175; complex64 512:
+//     198 / 194, 256: 190 / 127)
+template <typename T, int N>
+bool zw_takes(const PassArgs<T>& a, unsigned blocks) {
+    constexpr bool c128 = sizeof(T) == 8;
+    if constexpr (ZW<T, N>::B == 24) {
+        const unsigned slots = a.pipe_wgs, rounds = (blocks + slots - 1) / slots;
+        const bool full = 4 * (size_t)blocks > 3 * (size_t)rounds * slots;
+        const bool pinned = (a.flags & (F_IMPRINT | F_IMPRINT_MID | F_IMPRINT_NEXT)) != 0;
+        // passes that evaluate the interaction's potential
+        const bool pot = (a.load_mode == LOAD_PSI0 && (a.flags & F_VSTEP1)) || a.load_mode == LOAD_PART2 ||
+                         a.mid_mode == MID_VSTEP2 || a.mid_mode == MID_PART1 || a.mid_mode == MID_QF_VSTEP1 ||
+                         (a.mid_mode == MID_VSTEP3 && (a.flags & F_NEXT_VSTEP1));
+        if (pinned && !(c128 && full)) return false;
+        if (pot && a.ph.interactions == INT_ETF && !full) return false;
+        if (pot && a.ph.interactions == INT_UFG && (c128 ? 3 : 2) * blocks <= slots) return false;
+        if (c128 && 4 * blocks <= slots) return false;
+    }
+    return true;
+}
+
 // launches the z pass in the wave kernel when the length and the pass kind
 // have an instance; returns the workgroup count, 0 when the caller must use
 // the LDS-tile kernels
@@ -650,12 +691,7 @@ unsigned launch_zwave(const PassArgs<T>& a, hipStream_t s) {
         // compiled with the hook file; these kernels carry none of its code
         if (a.axis != 2 || a.nred > 3 || a.ph.modify) return 0;
         const unsigned blocks = (a.M + ZW<T, N>::PENCILS - 1) / ZW<T, N>::PENCILS;
-        // complex128 at 96 and 192 points holds 24 points per lane (256 VGPRs
-        // and some spills), so it pays once the workgroups reach more than half
-        // of the CUs: us per real-time step in LDS tiles / in waves 32x24x96
-        // 36 / 51, 64x64x192 84 / 88 (128 workgroups), 96^3 107 / 98 (144),
-        // 128x128x192 251 / 172, 192^3 551 / 395
-        if (sizeof(T) == 8 && ZW<T, N>::B > 16 && 4 * blocks <= a.pipe_wgs) return 0;
+        if (!zw_takes<T, N>(a, blocks)) return 0;
         const int shape = pass_shape(a.dir1, a.dir2);
         const int lm = (a.load_mode == LOAD_PLAIN && (a.flags & F_RED_POT)) ? LOAD_REDPOT : a.load_mode;
         const int mm = a.mid_mode;

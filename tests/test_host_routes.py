@@ -1,0 +1,72 @@
+"""Which kernels serve a call, on the host runtime: the rules that choose
+between forms of a pass, at both sides of their lines."""
+import pytest
+
+import host_runtime
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    return host_runtime.build(tmp_path_factory.mktemp("host"))
+
+
+ENGINE = """
+def engine(shape, ab=(1.0, 0.0), prec=E.C64, inter=E.CONTACT, vext=E.HARMONIC):
+    return E.Engine(shape, ab[0], ab[1], 0.01, 1.0, inter, vext, 0, prec)
+
+RT, IT = (1.0, 0.0), (0.0, 1.0)
+"""
+
+ZWAVE = ENGINE + """
+def z_passes(shape, ab, prec, inter, pinned=False, qf=0.0):
+    "(in waves, in LDS tiles) of the z passes of a run of three steps"
+    g = engine(shape, ab, prec, inter)
+    if pinned:
+        g.set_vortex(0.5, 0.5, 1)
+    if qf:
+        g.set_quantum_friction_coeff(qf)
+    names = launched(g.evolve_vortex if pinned else g.evolve_qf, 3)
+    g.close()
+    t = "f" if prec == E.C64 else "d"
+    waves = sum("zwave_kernelI%sLi%dE" % (t, shape[2]) in n for n in names)
+    tiles = sum("fft_pass_kernelI%sLi%dELb1E" % (t, shape[2]) in n for n in names)
+    return waves, tiles
+
+# z passes of three steps: open, then two per step in real time, four in
+# imaginary time (the last one's rescaling is not a z pass)
+N = {RT: 7, IT: 12}
+for ab in (RT, IT):
+    n = N[ab]
+    # contact: complex64 always, complex128 above 128 workgroups
+    assert z_passes((8, 12, 96), ab, E.C64, E.CONTACT) == (n, 0)
+    assert z_passes((64, 64, 192), ab, E.C128, E.CONTACT) == (0, n)
+    assert z_passes((96, 48, 192), ab, E.C128, E.CONTACT) == (n, 0)
+    # unitary gas: complex64 above 256, complex128 above 170; the passes
+    # without its potential as the contact ones
+    light = 1 if ab == RT else 3  # the last corrector end; every corrector end
+    assert z_passes((128, 128, 96), ab, E.C64, E.UFG) == (light, n - light)
+    assert z_passes((192, 96, 96), ab, E.C64, E.UFG) == (n, 0)
+    assert z_passes((96, 96, 96), ab, E.C128, E.UFG) == (light, n - light)
+    assert z_passes((128, 96, 96), ab, E.C128, E.UFG) == (n, 0)
+    # extended Thomas-Fermi: where the last round of two workgroups per CU is full
+    for shape, prec, waves in (((128, 128, 192), E.C128, True), ((128, 96, 192), E.C128, False),
+                               ((96, 96, 192), E.C128, False), ((128, 128, 192), E.C64, True),
+                               ((192, 192, 192), E.C64, False), ((8, 12, 96), E.C64, False)):
+        assert z_passes(shape, ab, prec, E.ETF) == ((n, 0) if waves else (light, n - light)), (shape, prec)
+    # pinned: only in complex128, there the same
+    for shape, prec, waves in (((128, 128, 192), E.C128, True), ((128, 96, 192), E.C128, False),
+                               ((128, 128, 192), E.C64, False), ((12, 8, 192), E.C64, False)):
+        pin = n - (light + 3 if ab == RT else 6)  # open and corrector ends that open a step; openings and re-imprints
+        got = z_passes(shape, ab, prec, E.CONTACT, pinned=True)
+        assert got == ((n, 0) if waves else (n - pin, pin)), (shape, prec, got, pin)
+# other lengths take waves whatever the pass
+for shape, precs in (((12, 8, 128), (E.C64, E.C128)), ((24, 8, 256), (E.C64, E.C128)),
+                     ((96, 96, 128), (E.C64, E.C128)), ((8, 12, 512), (E.C64,))):
+    for prec in precs:
+        for inter in (E.UFG, E.ETF, E.CONTACT):
+            assert z_passes(shape, RT, prec, inter, pinned=True) == (7, 0)
+"""
+
+
+def test_z_passes_of_24_points_per_lane(runtime):
+    host_runtime.run(runtime, ZWAVE)
