@@ -624,34 +624,64 @@ int fused_run(gpe_engine_s* e, int nt, hipStream_t s) {
 }
 
 // A small lattice's runs of steps in one kernel on one XCD (gpe_xcd.hpp): the
-// engine's own choice, made where no launcher variant was asked for.  The line
-// lies where one lattice alone on the GPU takes the passes' time, us per step
-// on one XCD / in passes: real time complex64 16^3 17.8 / 20.8, 32x32x24 23.2
-// / 32.1, 16x64x32 19.0 / 24.6, 24x48x32 33.1 / 26.6, complex128 16x24x32 22.9
-// / 25.7, 32x24x24 31.1 / 32.8; planes of 32 x 32: complex64 32^3 14.6 / 18.8,
-// complex128 24x32x32 18.0 / 18.6 (planes of 48 x 48, 27.9 / 27.2 and 30.4 /
-// 27.7, keep their passes); imaginary time complex64 32^3 25.3 / 38.4, 32x64x24
-// 48.9 / 47.9, complex128 48x24x16 31.0 / 34.8, 32^3 30.6 / 40.1.  Several
-// engines at once gain more (three 32^3 complex64: 4.9 / 14.9): each takes an
-// XCD of its own, and the host launches once per 256 steps.
-size_t xcd_most(const gpe_engine_s* e) {
-    const bool c64 = e->precision == GPE_PRECISION_C64;
-    if (e->beta != 0.0) return c64 ? 40960 : 32768;
-    return c64 ? 32768 : 24576;
+// engine's own choice, made where no launcher variant was asked for.  The lines
+// lie where one lattice alone on the GPU takes the passes' time, us per step on
+// one XCD / in passes, steps issued back to back (mean over four XCDs; where the
+// host waits for each run the passes take 4-20 us more a run):
+//   real time complex64, up to 32768 points: 32^3 (planes) 14.4 / 18.9, 64x64x8
+//     18.8 / 24.2, 8x64x64 17.3 / 24.2; 36864: 48x48x16 34.6 / 26.4, 24x24x64
+//     29.1 / 25.0; 24x32x32 (planes) 17.3 / 18.9, a run of one step 22.3 / 20.8
+//   real time complex128: a run spends 5-8 us on its launch and registration
+//     against the passes' two.  Four steps or more, up to 32768 points:
+//     64x24x16 21.6 / 23.5, 48x64x8 24.5 / 24.2, 8x64x64 20.3 / 26.4, 64x64x8
+//     21.1 / 22.7; 36864: 48x48x16 31.6 / 24.5, 24x24x64 25.7 / 26.0, 48x32x24
+//     39.3 / 33.9.  Fewer, up to 16384 points where
+//     z has 24 or more (runs of one step: 16x24x32 26.4 / 28.8, 16x32x24 34.8 /
+//     36.5; 18432: 12x48x32 32.0 / 29.6), else up to 4096 (16^3 21.5 / 26.8;
+//     4608: 48x12x8 26.1 / 24.2, 16384: 64x32x8 27.2 / 24.5).  Planes of
+//     32 x 32: four steps or more up to 16384 (16x32x32 18.0 / 19.2; 24x32x32 19.5 / 18.5),
+//     fewer up to 8192 (8x32x32 19.3 / 19.3; 12x32x32 23.0 / 19.5)
+//   imaginary time, complex128 up to 32768: 32^3 30.5 / 41.1; 36864: 48x48x16
+//     42.2 / 37.0, 24x24x64 33.7 / 41.1, 48x32x24 53.3 / 53.3; complex64 the same, and up to
+//     40960 where z has 24 or more: 24x48x32 38.6 / 42.5, 48x48x16 44.3 / 40.7
+// (planes of 48 x 48 keep their passes, 27.9 / 27.2 and 30.4 / 27.7; the other
+// interactions and potentials lie on the same sides).  Several engines at once
+// gain more (three 32^3 complex64: 4.9 / 14.9): each takes an XCD of its own,
+// and the host launches once per 256 steps.  Beside a large engine's run a
+// small one keeps its gain (256^3 complex64 in flight, 32^3: 20-22 us a step
+// in 256 steps, passes 20-23; 70-90 us a run of one step in both).
+constexpr int kXcdRun = 4;
+
+bool xcd_pays(const gpe_engine_s* e, int nt) {
+    const bool c64 = e->precision == GPE_PRECISION_C64, deep = e->nz >= 24, run = nt >= kXcdRun;
+    const bool plane = plane_selected(e, 0);
+    if (e->beta != 0.0) return e->n <= (c64 && deep ? 40960u : 32768u);
+    if (plane && e->nz != 32) return false;
+    if (c64) return e->n <= 32768 && !(plane && e->nx == 24 && !run);
+    if (plane) return e->n <= (run ? 16384u : 8192u);
+    return e->n <= (run ? 32768u : deep ? 16384u : 4096u);
 }
+
+// The grid and the queue assume the eight XCDs of 32 CUs of a whole MI355X; on
+// a partition of it, where no workgroup may ever see the wanted XCC_ID, the
+// engines keep their passes.
+constexpr unsigned kXcds = 8, kXcdCus = 32;
 
 bool xcd_lattice(const gpe_engine_s* e) {
-    return e->batch == 1 && xcd_length(e->nx) && xcd_length(e->ny) && xcd_length(e->nz) && e->n <= 40960 &&
-           !e->uses_hooks && e->interactions != INT_DIPOLAR;
+    return e->cus == (int)(kXcds * kXcdCus) && e->batch == 1 && xcd_length(e->nx) && xcd_length(e->ny) &&
+           xcd_length(e->nz) && e->n <= 40960 && !e->uses_hooks && e->interactions != INT_DIPOLAR;
 }
 
-bool xcd_selected(const gpe_engine_s* e, int pin) {
-    if (!e->xcdq || !(e->beta != 0.0 ? e->xcd_it : e->xcd_rt) || e->n > xcd_most(e) || pin != 0 || e->qf != 0.0 || e->use_graph || e->prof_class >= 0)
-        return false;
-    if (plane_selected(e, pin) && e->nz != 32) return false;
+// a run of nt steps can go to one XCD
+bool xcd_can(const gpe_engine_s* e, int pin, int nt) {
+    if (!e->xcdq || pin != 0 || e->qf != 0.0 || e->use_graph || e->prof_class >= 0 || !xcd_pays(e, nt)) return false;
     // a captured launch would be replayed with the queue words of its first run
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(e->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+}
+
+bool xcd_selected(const gpe_engine_s* e, int pin, int nt) {
+    return (e->beta != 0.0 ? e->xcd_it : e->xcd_rt) && xcd_can(e, pin, nt);
 }
 
 // nt steps, in launches of at most 256 so that no single kernel runs for long
@@ -668,17 +698,16 @@ int xcd_run(gpe_engine_s* e, int nt) {
         *lo[a] = (const cplx<T>*)e->twlo[a];
     }
     // a workgroup for every 512 points, at most one for each CU of the XCD
-    const unsigned xcds = e->cus >= 256 ? 8u : 1u;
-    g.xcd = e->xcd_home % xcds;
-    g.want = std::min((unsigned)e->cus / xcds, (unsigned)((e->n + 511) / 512));
+    g.xcd = e->xcd_home % kXcds;
+    g.want = std::min(kXcdCus, (unsigned)((e->n + 511) / 512));
     constexpr int kChunk = 256;
     for (int done = 0; done < nt; done += kChunk) {
         g.nt = std::min(kChunk, nt - done);
         g.q = e->xcdq + (e->xcd_flip ? kXqWords : 0);
         g.qnext = e->xcdq + (e->xcd_flip ? 0 : kXqWords);
         e->xcd_flip = !e->xcd_flip;
-        if (plane_selected(e, 0)) launch_xcd_plane32<T>(g, xcds * g.want, e->stream);
-        else if (!launch_xcd<T>(e->nz, g, e->beta != 0.0, xcds * g.want, e->stream)) return GPE_ERR_ARG;
+        if (plane_selected(e, 0)) launch_xcd_plane32<T>(g, kXcds * g.want, e->stream);
+        else if (!launch_xcd<T>(e->nz, g, e->beta != 0.0, kXcds * g.want, e->stream)) return GPE_ERR_ARG;
     }
     HIP_TRY(hipGetLastError());
     return 0;
@@ -687,7 +716,7 @@ int xcd_run(gpe_engine_s* e, int nt) {
 template <typename T>
 int evolve_t(gpe_engine_s* e, int nt, double* mu, int pin, bool mid_pin) {
     if (nt <= 0) return 0;
-    if (xcd_selected(e, pin)) {
+    if (xcd_selected(e, pin, nt)) {
         if (int r = xcd_run<T>(e, nt)) return r;
         e->it = e->it + (unsigned)nt;
         if (e->beta != 0.0 && mu) {
@@ -936,6 +965,12 @@ int create_impl(gpe_engine_s** out, const gpe_config_t* cfg, double alpha, doubl
         delete e;
         return code;
     };
+    {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+            e->cus = cus;
+    }
     hipError_t err;
 #define ALLOC(ptr, bytes)                               \
     err = hipMalloc((void**)&(ptr), (bytes));           \
@@ -983,12 +1018,6 @@ int create_impl(gpe_engine_s** out, const gpe_config_t* cfg, double alpha, doubl
     int r = (e->precision == GPE_PRECISION_C64) ? upload_static_tables<float>(e) : upload_static_tables<double>(e);
     if (!r) r = upload_potential_any(e);
     if (r) return fail(r);
-    {
-        int dev = 0, cus = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
-            e->cus = cus;
-    }
     e->variant = default_variant(e);
     *out = e;
     return 0;
@@ -2153,7 +2182,7 @@ int autotune_t(gpe_engine_s* e, int steps, int* chosen) {
     e->xcd_it = e->xcd_rt = true;
     if (!err && e->xcdq) {
         e->beta = 0.0;
-        bool win = xcd_selected(e, 0);
+        bool win = xcd_selected(e, 0, steps);
         if (win) {
             err = xcd_run<T>(e, 1);
             (void)hipEventRecord(t0, e->stream);

@@ -70,3 +70,52 @@ for shape, precs in (((12, 8, 128), (E.C64, E.C128)), ((24, 8, 256), (E.C64, E.C
 
 def test_z_passes_of_24_points_per_lane(runtime):
     host_runtime.run(runtime, ZWAVE)
+
+
+XCD = ENGINE + """
+def one_xcd(shape, ab, prec, nt, inter=E.CONTACT, prepare=None):
+    g = engine(shape, ab, prec, inter, E.COSINE)
+    if prepare:
+        prepare(g)
+    names = launched(g.evolve_qf, nt)
+    g.close()
+    on = any("xcd_" in n for n in names)
+    assert on == all("xcd_" in n for n in names), names
+    return on
+
+# (points' sides of the lines: shape, time, precision, steps -> one XCD)
+for shape, ab, prec, nt, want in [
+        ((32, 32, 32), RT, E.C64, 1, True), ((64, 64, 8), RT, E.C64, 1, True), ((24, 24, 64), RT, E.C64, 20, False),
+        ((24, 32, 32), RT, E.C64, 3, False), ((24, 32, 32), RT, E.C64, 4, True),
+        ((16, 24, 32), RT, E.C128, 1, True), ((16, 32, 24), RT, E.C128, 3, True), ((12, 24, 64), RT, E.C128, 3, False),
+        ((12, 24, 64), RT, E.C128, 4, True), ((16, 16, 16), RT, E.C128, 1, True), ((48, 12, 8), RT, E.C128, 3, False),
+        ((48, 12, 8), RT, E.C128, 4, True), ((64, 64, 8), RT, E.C128, 4, True), ((24, 24, 64), RT, E.C128, 20, False),
+        ((8, 32, 32), RT, E.C128, 1, True), ((12, 32, 32), RT, E.C128, 3, False), ((16, 32, 32), RT, E.C128, 4, True),
+        ((24, 32, 32), RT, E.C128, 20, False), ((12, 48, 48), RT, E.C64, 20, False),
+        ((32, 32, 32), IT, E.C128, 1, True), ((48, 24, 32), IT, E.C128, 20, False), ((48, 24, 32), IT, E.C64, 1, True),
+        ((48, 48, 16), IT, E.C64, 20, False), ((48, 48, 16), (0.6, 0.3), E.C64, 20, False),
+        ((32, 32, 32), (0.6, 0.3), E.C64, 1, True), ((96, 8, 8), RT, E.C64, 20, False)]:
+    assert one_xcd(shape, ab, prec, nt) == want, (shape, ab, prec, nt)
+for inter in (E.UFG, E.ETF):
+    assert one_xcd((16, 16, 16), RT, E.C64, 5, inter)
+
+# what keeps the passes, and what does not
+SMALL = ((16, 24, 32), RT, E.C64, 20)
+assert one_xcd(*SMALL)
+assert not one_xcd(*SMALL, prepare=lambda g: g.set_variant(0))
+assert not one_xcd(*SMALL, prepare=lambda g: g.set_quantum_friction_coeff(0.1))
+H.hh_capture(1)
+assert not one_xcd(*SMALL)
+H.hh_capture(0)
+# a partition of the card: fewer CUs, or another count, than eight XCDs of 32
+for cus in (32, 64, 128, 255, 304):
+    H.hh_cus(cus)
+    assert not one_xcd(*SMALL), cus
+    assert not one_xcd((32, 32, 32), IT, E.C128, 20), cus
+H.hh_cus(256)
+assert one_xcd(*SMALL)
+"""
+
+
+def test_runs_on_one_xcd(runtime):
+    host_runtime.run(runtime, XCD)
