@@ -251,9 +251,11 @@ const char *gpe_build_info(void);
  * times
  * `steps` real-time steps per choice on the current state (restored
  * afterwards) and keeps the fastest.  An engine whose variant was never set
- * runs a small lattice (lengths up to 64, about 32 k points, built-in physics,
- * no pinning or friction) in one kernel per 256 steps, with the same results;
- * set_variant selects the passes, autotune times both. */
+ * runs a small lattice (lengths up to 64, up to about 32 k points, built-in
+ * physics, no pinning or friction) in one kernel per 256 steps, with the same
+ * results.  set_variant selects the passes for both time modes; autotune times
+ * that kernel too, on real-time steps, and takes it back where it wins, unless
+ * friction, graphs or profiling are on.  Imaginary time stays as set. */
 int gpe_engine_autotune(gpe_engine_t e, int steps, int *variant);
 int gpe_engine_set_variant(gpe_engine_t e, int variant);
 /* 1: an evolve call of 3 or more steps replays HIP graphs of the open pass,

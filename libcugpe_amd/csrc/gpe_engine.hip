@@ -109,8 +109,8 @@ struct gpe_engine_s {
 
     // runs of a small lattice on one XCD (gpe_xcd.hpp): the queue words of two
     // launches (null: not such a lattice), which of them is next, the XCD, and
-    // whether imaginary- and real-time runs may take it (cleared by a launcher
-    // variant set by hand; the autotuner decides for real time)
+    // whether imaginary- and real-time runs may take it (both cleared by a launcher
+    // variant set by hand; a timing by the autotuner decides for real time)
     unsigned* xcdq = nullptr;
     unsigned xcd_home = 0;
     bool xcd_flip = false, xcd_it = true, xcd_rt = true;
@@ -2177,25 +2177,24 @@ int autotune_t(gpe_engine_s* e, int steps, int* chosen) {
         }
     }
     // a small lattice's real-time run on one XCD, kept where it beats the variant
-    // chosen, whose passes serve the runs it does not cover
+    // chosen, whose passes serve the runs it does not cover.  Only a timing
+    // changes the route: not while friction, graphs or profiling keep the passes,
+    // and not the route of imaginary time, which is not timed.
     e->variant = best;
-    e->xcd_it = e->xcd_rt = true;
     if (!err && e->xcdq) {
+        const int xs = std::max(steps, kXcdRun);
         e->beta = 0.0;
-        bool win = xcd_selected(e, 0, steps);
-        if (win) {
+        if (xcd_can(e, 0, xs)) {
             err = xcd_run<T>(e, 1);
             (void)hipEventRecord(t0, e->stream);
-            if (!err) err = xcd_run<T>(e, steps);
+            if (!err) err = xcd_run<T>(e, xs);
             (void)hipEventRecord(t1, e->stream);
             float ms = 0.f;
             const hipError_t h = hipEventSynchronize(t1);
             if (!err && h != hipSuccess) err = (int)h;
-            win = !err && hipEventElapsedTime(&ms, t0, t1) == hipSuccess && ms < best_ms;
-            if (win) best_ms = ms;
+            if (!err && hipEventElapsedTime(&ms, t0, t1) == hipSuccess) e->xcd_rt = ms * steps < best_ms * xs;
         }
         e->beta = beta;
-        e->xcd_rt = win;
     }
     (void)hipMemcpyAsync(e->A, save, bytes, hipMemcpyDeviceToDevice, e->stream);
     (void)hipStreamSynchronize(e->stream);

@@ -119,3 +119,51 @@ assert one_xcd(*SMALL)
 
 def test_runs_on_one_xcd(runtime):
     host_runtime.run(runtime, XCD)
+
+
+AUTOTUNE = ENGINE + """
+def on(g, n=20):
+    return all("xcd_" in k for k in launched(g.evolve_qf, n))
+
+def other(g, rt):
+    g.set_ite_evolution() if not rt else g.set_rte_evolution()
+
+H.hh_cost(b"xcd_", float(XCD_MS))
+fast = XCD_MS < 0.1
+for prec, shape in ((E.C64, (16, 24, 32)), (E.C128, (32, 32, 16))):
+    # never set: imaginary time keeps its route, real time the faster one
+    g = engine(shape, RT, prec)
+    assert on(g)
+    g.autotune(3)
+    assert on(g) == fast
+    g.set_ite_evolution()
+    assert on(g)
+    g.close()
+    # set by hand: passes; a timing brings back real time, where it wins
+    g = engine(shape, RT, prec)
+    g.set_variant(2)
+    g.set_ite_evolution()
+    g.autotune(3)
+    assert not on(g)
+    g.set_rte_evolution()
+    assert on(g) == fast
+    g.close()
+    # not timed: the route stays as it was
+    for start in (None, 2):
+        for busy, quiet in ((lambda g: g.set_quantum_friction_coeff(0.1), lambda g: g.set_quantum_friction_coeff(0.0)),
+                            (lambda g: g.set_graph(True), lambda g: g.set_graph(False)),
+                            (lambda g: g.profile(1), lambda g: g.profile(1, False))):
+            g = engine(shape, RT, prec)
+            if start is not None:
+                g.set_variant(start)
+            busy(g)
+            g.autotune(3)
+            quiet(g)
+            assert on(g) == (start is None), (start, prec)
+            g.close()
+"""
+
+
+@pytest.mark.parametrize("ms", [0.001, 1000.0])
+def test_autotune_changes_a_route_only_by_a_timing(runtime, ms):
+    host_runtime.run(runtime, "XCD_MS = %r\n" % ms + AUTOTUNE)
