@@ -294,17 +294,21 @@ __device__ __forceinline__ void dft3(cplx<T>* v) {
     constexpr double hd = 0.86602540378443864676;  // sqrt(3)/2
     cplx<T> t1 = cadd(v[1], v[2]), t2 = csub(v[1], v[2]);
     cplx<T> m = mk(v[0].x - (T)0.5 * t1.x, v[0].y - (T)0.5 * t1.y);
-    cplx<T> ht2;
     if constexpr (sizeof(T) == 4) {
         constexpr float hh = (float)hd, hl = (float)(hd - (double)hh);
-        ht2 = mk(fmaf(t2.x, hh, t2.x * hl), fmaf(t2.y, hh, t2.y * hl));
+        const cplx<T> ht2 = mk(fmaf(t2.x, hh, t2.x * hl), fmaf(t2.y, hh, t2.y * hl));
+        const cplx<T> it2 = mk(-(T)S * ht2.y, (T)S * ht2.x);
+        v[0] = cadd(v[0], t1);
+        v[1] = cadd(m, it2);
+        v[2] = csub(m, it2);
     } else {
-        ht2 = mk((T)hd * t2.x, (T)hd * t2.y);
+        // one rounding, as the compiler makes of a product and a sum where it
+        // contracts across expressions: lengths up to 64 are compiled without
+        constexpr double h = S * hd;
+        v[0] = cadd(v[0], t1);
+        v[1] = mk(fma(-h, t2.y, m.x), fma(h, t2.x, m.y));
+        v[2] = mk(fma(h, t2.y, m.x), fma(-h, t2.x, m.y));
     }
-    cplx<T> it2 = mk(-(T)S * ht2.y, (T)S * ht2.x);
-    v[0] = cadd(v[0], t1);
-    v[1] = cadd(m, it2);
-    v[2] = csub(m, it2);
 }
 
 template <int S, typename T>
