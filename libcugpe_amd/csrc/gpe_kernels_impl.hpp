@@ -204,19 +204,22 @@ __device__ __forceinline__ int plaquette(const Corner& a, const Corner& b, const
     return (quarter_turns(a, b) + quarter_turns(b, c) + quarter_turns(c, d) + quarter_turns(d, a)) / 4;
 }
 
-// A thread walks kWindRun points along x, so every corner is loaded, classified
-// and located once and serves the planes on both sides of it (12 loads, 12
-// classifications and two integer divisions per point before: 128^3 complex128
-// 32.7 -> 23.8 us for the count).  w may be null: the count alone.
-constexpr unsigned kWindRun = 8;
-template <typename T>
+// A thread walks RUN points along x, so every corner is loaded, classified
+// and located once and serves the planes on both sides of it.  w may be null:
+// the count alone.  A run is a serial chain of loads, so it pays once its threads
+// fill the chip (256 CUs of 1024): us of a count at a run of 1 / of 8, complex128:
+// 32^3 26.1 / 36.9, 64^3 27.8 / 37.0, 128x128x64 (131072 threads of 8) 36.2 /
+// 38.2, 128^3 (262144) 52.6 / 45.8, 256^3 257 / 199 (26.4, 29.0, 39.9, 56.0 and 284
+// with 12 loads, 12 classifications and two integer divisions per point).
+constexpr unsigned kWindRun = 8, kWindThreads = 196608;
+template <typename T, unsigned RUN>
 __global__ __launch_bounds__(kThreads) void windings_kernel(const cplx<T>* __restrict__ A, int nx, int ny, int nz,
                                                             double rho_min, int8_t* __restrict__ w,
                                                             double* __restrict__ partials) {
     __shared__ double red[kThreads / 64];
     const unsigned ux = (unsigned)nx, uy = (unsigned)ny, uz = (unsigned)nz, plane = uy * uz;
     const unsigned n = ux * plane;
-    const unsigned runs = (ux + kWindRun - 1) / kWindRun;
+    const unsigned runs = (ux + RUN - 1) / RUN;
     double cnt = 0.0;
     const unsigned stride = gridDim.x * kThreads;
     // plane runs <= n / 8 + plane < 2^31, so the index does not wrap within one stride past it
@@ -225,7 +228,7 @@ __global__ __launch_bounds__(kThreads) void windings_kernel(const cplx<T>* __res
         const unsigned iy = r / uz, iz = r - iy * uz;
         const unsigned jy = (iy + 1 == uy) ? 0 : iy + 1, jz = (iz + 1 == uz) ? 0 : iz + 1;
         const unsigned o10 = jy * uz + iz, o01 = iy * uz + jz, o11 = jy * uz + jz;
-        const unsigned x0 = run * kWindRun, x1 = x0 + kWindRun < ux ? x0 + kWindRun : ux;
+        const unsigned x0 = run * RUN, x1 = x0 + RUN < ux ? x0 + RUN : ux;
         const cplx<T>* p = A + (size_t)x0 * plane;
         Corner a00 = corner(p[r], rho_min), a10 = corner(p[o10], rho_min), a01 = corner(p[o01], rho_min),
                a11 = corner(p[o11], rho_min);
@@ -306,8 +309,14 @@ int launch_norm_partials_impl(const cplx<T>* A, unsigned n, double gamma, double
 template <typename T>
 int launch_windings_impl(const cplx<T>* A, int nx, int ny, int nz, double rho_min, int8_t* w, double* partials,
                          hipStream_t s) {
-    const int nb = reduce_grid((unsigned)ny * nz * (((unsigned)nx + kWindRun - 1) / kWindRun));
-    hipLaunchKernelGGL((windings_kernel<T>), dim3(nb), dim3(kThreads), 0, s, A, nx, ny, nz, rho_min, w, partials);
+    const unsigned plane = (unsigned)ny * nz, runs = ((unsigned)nx + kWindRun - 1) / kWindRun;
+    if (plane * runs >= kWindThreads) {
+        const int nb = reduce_grid(plane * runs);
+        hipLaunchKernelGGL((windings_kernel<T, kWindRun>), dim3(nb), dim3(kThreads), 0, s, A, nx, ny, nz, rho_min, w, partials);
+        return nb;
+    }
+    const int nb = reduce_grid(plane * (unsigned)nx);
+    hipLaunchKernelGGL((windings_kernel<T, 1>), dim3(nb), dim3(kThreads), 0, s, A, nx, ny, nz, rho_min, w, partials);
     return nb;
 }
 

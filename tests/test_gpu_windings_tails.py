@@ -1,5 +1,5 @@
 """Vortex detection at the ends of its runs along x: lengths of 8 (one run), 12
-(a run of 8 and a rest of 4) and more, against the oracle bit for bit, and the
+(a run of 8 and a rest of 4) and more, with runs of 1 (small lattices) and 8, against the oracle bit for bit, and the
 count alone, which takes no array."""
 import numpy as np
 import pytest
@@ -22,7 +22,7 @@ def state(shape, seed):
 
 @pytest.mark.parametrize("prec", [E.C128, E.C64])
 @pytest.mark.parametrize("shape", [(8, 8, 8), (8, 24, 16), (12, 8, 16), (12, 12, 12), (12, 64, 48), (16, 12, 8),
-                                   (24, 16, 12), (48, 8, 8)])
+                                   (24, 16, 12), (48, 8, 8), (8, 512, 384), (12, 256, 512)])
 def test_windings_and_count(oracle, shape, prec):
     print("[gpu-case] windings", shape, prec, flush=True)
     psi = state(shape, 5)

@@ -167,3 +167,17 @@ for prec, shape in ((E.C64, (16, 24, 32)), (E.C128, (32, 32, 16))):
 @pytest.mark.parametrize("ms", [0.001, 1000.0])
 def test_autotune_changes_a_route_only_by_a_timing(runtime, ms):
     host_runtime.run(runtime, "XCD_MS = %r\n" % ms + AUTOTUNE)
+
+
+WINDINGS = ENGINE + """
+for shape, run in (((8, 8, 8), 1), ((64, 64, 64), 1), ((128, 128, 64), 1), ((128, 128, 128), 8), ((12, 256, 512), 8)):
+    for prec in (E.C64, E.C128):
+        g = engine(shape, prec=prec)
+        names = [n for n in launched(g.detect_vortices, 0.1, False) if "windings" in n]
+        assert len(names) == 1 and "Lj%dE" % run in names[0], (shape, names)
+        g.close()
+"""
+
+
+def test_vortex_detection_runs(runtime):
+    host_runtime.run(runtime, WINDINGS)
