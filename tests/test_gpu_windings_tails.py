@@ -22,7 +22,7 @@ def state(shape, seed):
 
 @pytest.mark.parametrize("prec", [E.C128, E.C64])
 @pytest.mark.parametrize("shape", [(8, 8, 8), (8, 24, 16), (12, 8, 16), (12, 12, 12), (12, 64, 48), (16, 12, 8),
-                                   (24, 16, 12), (48, 8, 8), (8, 512, 384), (12, 256, 512)])
+                                   (24, 16, 12), (48, 8, 8), (8, 512, 512), (12, 256, 512)])
 def test_windings_and_count(oracle, shape, prec):
     print("[gpu-case] windings", shape, prec, flush=True)
     psi = state(shape, 5)
