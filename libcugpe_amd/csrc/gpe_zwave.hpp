@@ -618,8 +618,13 @@ __device__ __forceinline__ void zwave_tile(const PassArgs<T>& a, const TwE<T>* t
     }
 }
 
+// At 512 points a pass is 0.2-0.4 MB of code, more than the instruction cache,
+// and where it lies is worth up to 9% of the pass (Vstep2 899 or 979 us at 512^3
+// with the same instructions 0x1100 bytes apart; whole steps 4410 and 4476 us).
+// Entries at multiples of 1 KiB measured best (4368; 4 KiB 4465, 64 KiB 4455).
 template <typename T, int N, int SHAPE, int LM, int MM>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(zw_waves<T, N, SHAPE, LM, MM>())))
+__attribute__((aligned(N > 256 ? 1024 : 256)))
 void zwave_kernel(const PassArgs<T> a) {
     __shared__ ZwLds<T, N> L;
     zwave_stage<T, N>(a, L.tw, L.vz);
